@@ -74,7 +74,9 @@ typedef enum rf_w8a16_status {
 #define RF_W8A16_KERNEL_GEMV 1 /* decode GEMV / skinny GEMM, M <= 64 (AUTO: M <= 16, M <= 24
                                   with N*K < 2^25, M <= 28 with N*K <= 2^24,
                                   M <= 32 with N*K <= 2^23 or N <= 2048 and
-                                  N*K <= 2^24; W4A16: M <= 64)                */
+                                  N*K <= 2^24; W4A16: M <= 16, M <= 24 with
+                                  N*K <= 2^24, M <= 32 with N*K <= 2^22, M <= 64
+                                  with K < 1024)                              */
 #define RF_W8A16_KERNEL_GEMM 2 /* prefill GEMM: x tiles staged in LDS by DMA, int8 weight
                                   tiles dequantized into fp16 MFMA operands (from
                                   registers on the large tiles, from LDS on the others) */
@@ -298,7 +300,8 @@ size_t rf_w4a16_workspace_bytes_multi(int64_t M, const int64_t* Ns, int32_t coun
  * scale [N]) or 32 / 64 / 128 (scale [K/group_size][N], 16-byte aligned).
  * kernel, workspace and stream as for rf_w8a16_linear; the int4 GEMM has no
  * 64-bit-address kernel and returns RF_W8A16_EKERNEL where a tile's rows
- * (up to 128 rows of ldx halves) span 4 GB or more. */
+ * (up to 128 rows of ldx halves) span 4 GB or more (AUTO then runs the GEMV
+ * where M <= 64). */
 int rf_w4a16_linear(const void* x, int64_t ldx, const void* w_packed, const void* scale,
                     int32_t group_size, const void* bias, void* y, int64_t ldy, int64_t M,
                     int64_t N, int64_t K, int32_t kernel, void* workspace, size_t workspace_bytes,

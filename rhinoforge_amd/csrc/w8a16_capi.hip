@@ -161,8 +161,35 @@ int auto_kernel(int64_t M, int64_t N, int64_t K) {
   return RF_W8A16_KERNEL_GEMM;
 }
 
-// W4A16 keeps the GEMV up to its M = 64 limit (its GEMM has no small tiles).
-int auto_kernel_int4(int64_t M) { return M <= 64 ? RF_W8A16_KERNEL_GEMV : RF_W8A16_KERNEL_GEMM; }
+// W4A16: the GEMV up to M = 16; from M = 17 the GEMM's tiles of 128-wide K
+// blocks win on every launch but small ones, where their pipeline fill shows:
+// N*K <= 2^24 up to M = 24 (4096 x 4096 at M 24: GEMV 9.4, GEMM 9.6 us), N*K
+// <= 2^22 up to M = 32 (1024 x 4096: 8.0 against 8.5 us) and K < 1024 up to M
+// = 64 (MI355X, graph-timed, 600 MB of rotated weights).  A launch whose row
+// stride the GEMM's 32-bit tile offsets cannot address stays on the GEMV
+// wherever that can (M <= 64).
+int auto_kernel_int4(int64_t M, int64_t N, int64_t K) {
+  if (M <= 16) return RF_W8A16_KERNEL_GEMV;
+  const int64_t nk = N * K;
+  if ((M <= 24 && nk <= ((int64_t)1 << 24)) || (M <= 32 && nk <= ((int64_t)1 << 22)) ||
+      (M <= 64 && K < 1024))
+    return RF_W8A16_KERNEL_GEMV;
+  return RF_W8A16_KERNEL_GEMM;
+}
+
+// The kernel an AUTO call of packed int4 weights runs at row stride ldx.
+int auto_kernel_int4_at(int64_t M, const int* Ns, int count, int64_t K, int64_t ldx,
+                        const rf::DeviceInfo& dev) {
+  int64_t ntotal = 0;
+  for (int i = 0; i < count; ++i) ntotal += Ns[i];
+  const int k = auto_kernel_int4(M, ntotal, K);
+  const bool gemv_ok = M <= 64 && rf::gemv_offsets_fit(M, ldx);
+  if (k == RF_W8A16_KERNEL_GEMV) return gemv_ok ? k : RF_W8A16_KERNEL_GEMM;
+  if (gemv_ok && !rf::gemm_offsets_fit(rf::plan_gemm((int)M, Ns, count, (int)K, dev, true), ldx,
+                                       (int)K, true))
+    return RF_W8A16_KERNEL_GEMV;
+  return k;
+}
 
 }  // namespace
 
@@ -335,7 +362,7 @@ int rf_w8a16_plan(int64_t M, const int64_t* Ns, int32_t count, int64_t K, int32_
     if (st != RF_W8A16_OK) return st;
   }
   if (kernel == RF_W8A16_KERNEL_AUTO) {
-    kernel = int4 ? auto_kernel_int4(M) : auto_kernel(M, ntotal, K);
+    kernel = int4 ? auto_kernel_int4_at(M, n32, count, K, K, dev) : auto_kernel(M, ntotal, K);
     if (kernel == RF_W8A16_KERNEL_GEMV && !rf::gemv_offsets_fit(M, K))
       kernel = RF_W8A16_KERNEL_GEMM;  // the fallback the compute entry points take
   }
@@ -633,11 +660,9 @@ int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs
   if (st != RF_W8A16_OK) return st;
   if (!dev.gfx950) return RF_W8A16_EDEVICE;
 
-  if (kernel == RF_W8A16_KERNEL_AUTO) {
-    kernel = auto_kernel_int4(M);
-    if (kernel == RF_W8A16_KERNEL_GEMV && !rf::gemv_offsets_fit(M, ldx))
-      kernel = RF_W8A16_KERNEL_GEMM;
-  }
+  int n32[RF_W8A16_MAX_PROJ];
+  for (int i = 0; i < count; ++i) n32[i] = (int)projs[i].N;
+  if (kernel == RF_W8A16_KERNEL_AUTO) kernel = auto_kernel_int4_at(M, n32, count, K, ldx, dev);
   if (kernel != RF_W8A16_KERNEL_GEMV && kernel != RF_W8A16_KERNEL_GEMM) return RF_W8A16_EINVAL;
   if (kernel == RF_W8A16_KERNEL_GEMV && (M > 64 || !rf::gemv_offsets_fit(M, ldx)))
     return RF_W8A16_EKERNEL;
@@ -651,7 +676,6 @@ int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs
   pr.nproj = count;
   pr.wf = group_size ? rf::kWfInt4Grp : rf::kWfInt4;
   pr.gshift = group_size == 128 ? 2 : group_size == 64 ? 1 : 0;
-  int n32[RF_W8A16_MAX_PROJ];
   for (int i = 0; i < count; ++i) {
     rf::Projection& d = pr.proj[i];
     d.w = static_cast<const uint8_t*>(projs[i].w_packed);
@@ -660,7 +684,6 @@ int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs
     d.y = static_cast<_Float16*>(projs[i].y);
     d.ldy = projs[i].ldy;
     d.N = (int)projs[i].N;
-    n32[i] = d.N;
   }
   auto workspace_ok = [&](size_t extra) {
     return workspace && workspace_bytes >= RF_W8A16_WS_COUNTER_BYTES + extra &&

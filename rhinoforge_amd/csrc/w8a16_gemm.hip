@@ -136,6 +136,12 @@ __device__ __forceinline__ void dma16s(uint32_t voff, const void* sbase, uint32_
 // 32-lane group cover distinct LDS banks (64 or 128 banks of 4 bytes).
 __device__ __forceinline__ int a_swizzle(int r) { return (r & 7) ^ (((r >> 3) & 1) * 5); }
 
+// 128-wide K blocks: there the second 16 lanes of a fragment read are at
+// chunk ^ 4, so chunks are stored with bits 1 and 2 of their index exchanged
+// (its own inverse), which makes that slot ^ 2 again.  (A read of the plain
+// order runs at half the rate: 290 against 494 GB/s per CU, eight wavefronts.)
+__device__ __forceinline__ int a_chunk128(int c) { return (c & 1) | ((c & 2) << 1) | ((c & 4) >> 1); }
+
 // Buffer resource over the split-K partials; accesses use sc1 (device-scope
 // coherent: written through / re-fetched past the issuing XCD's L2, the
 // same instructions as relaxed agent-scope atomic stores and loads).
@@ -219,28 +225,41 @@ __device__ __forceinline__ void store_tile(const TileTarget& t, const floatx4 (&
 // launch of one tile per CU still keeps two wavefronts on every SIMD, each
 // with the instruction mix of the one-group tile.  At the end group 1 hands
 // its accumulators to group 0 through LDS, which adds them (fixed order).
+//
+// KB: 64-wide K blocks per stage (int4 only: 2, one whole TILE16X128_I4 tile
+// per strip and stage; a.kblocks and a.kb_per_split then count 128-wide
+// blocks).  The A tile is two 64-wide sub-tiles of the layout above, one
+// behind the other; lane (g = l/16, c = l%16) reads its strip's 16 bytes with
+// one LDS read, dword j holding positions 32g + 8j .. +7 of the block, so A
+// fragment j is chunk 4(g%2) + j of sub-tile g/2.  A strip is 1 KB per stage
+// instead of 512 B, so 64-column tiles (whose half tiles are less than one
+// DMA round of four wavefronts) can be staged, at half the barriers.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int OCC, int WF = kWfInt8,
-          bool IL = false, bool BR = false, int KG = 1>
+          bool IL = false, bool BR = false, int KG = 1, int KB = 1>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64 * KG) __attribute__((amdgpu_waves_per_eu(OCC * WAVES_M * WAVES_N * KG / 4, 8)))
 void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int A_BYTES = BM * 128;
+  constexpr int A_SUB = BM * 128;       // one 64-wide sub-tile of A
+  constexpr int A_BYTES = KB * A_SUB;
   constexpr int B_TILES = BN / 16;
-  constexpr int B_STRIP = WF ? kTileBytes / 2 : kTileBytes;  // per strip and K block
+  constexpr int B_STRIP = WF && KB == 1 ? kTileBytes / 2 : kTileBytes;  // per strip and stage
   constexpr int B_BYTES = B_TILES * B_STRIP;
   constexpr bool GS = WF == kWfInt4Grp;
-  constexpr int S_BYTES = GS ? 1024 : 0;  // one wavefront DMA of scale rows
-  static_assert(!GS || 2 * BN * 2 <= S_BYTES, "two scale rows of BN fp16 fit one DMA");
+  static_assert(KB == 1 || (KB == 2 && WF != kWfInt8 && !IL && !BR),
+                "two K blocks per stage: int4, plain schedule");
+  // Scale rows of a stage (at most two per 64-wide block), copied by wavefront 0.
+  constexpr int S_LOADS = GS ? (2 * KB * BN * 2 + 1023) / 1024 : 0;
+  constexpr int S_BYTES = S_LOADS * 1024;
   // BR: each wavefront loads its own B strips straight into registers (in a
   // 1 x N grid no two wavefronts share a strip, so staging B in LDS only adds
   // a DMA write and a read per byte); LDS then holds A (and scales) only.
   constexpr int S_OFF = A_BYTES + (BR ? 0 : B_BYTES);
   constexpr int SUB = S_OFF + S_BYTES;  // one K block's LDS
   constexpr int STAGE = KG * SUB;       // one block per K group
-  static_assert(KG == 1 || (KG == 2 && !IL && WF == kWfInt8),
-                "two K groups: int8, plain schedule");
+  static_assert(KG == 1 || (KG == 2 && !IL && (WF == kWfInt8 || KB == 2)),
+                "two K groups: int8 or 128-wide int4 blocks, plain schedule");
   constexpr int A_LOADS = A_BYTES / (NT * 16);
   constexpr int B_LOADS = BR ? 0 : B_BYTES / (NT * 16);
   constexpr int LOADS = A_LOADS + B_LOADS;
@@ -282,9 +301,11 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
 #pragma unroll
   for (int i = 0; i < A_LOADS; ++i) {
     const int p = (wave * A_LOADS + i) * 64 + lane;
-    const int row = p >> 3;
-    const int chunk = (p & 7) ^ a_swizzle(row);
-    acol[i] = chunk * 8;
+    const int sub = KB == 1 ? 0 : p / (BM * 8);
+    const int row = (p - sub * BM * 8) >> 3;
+    const int slot = (p & 7) ^ a_swizzle(row);
+    const int chunk = KB == 2 ? a_chunk128(slot) : slot;
+    acol[i] = sub * 64 + chunk * 8;
     const int r = min(m0 + row, a.M - 1) - m0;
     arow_off[i] = (uint32_t)((int64_t)r * a.ldx * 2);
     aoff[i] = arow_off[i] + acol[i] * 2;
@@ -292,7 +313,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   uint32_t boff[B_LOADS > 0 ? B_LOADS : 1];
 #pragma unroll
   for (int i = 0; i < B_LOADS; ++i) {
-    if (WF) {
+    if (WF && KB == 1) {
       // 16-byte chunk p of the stage's B: strip p/32, chunk p%32 of its half tile
       const int p = (wave * B_LOADS + i) * 64 + lane;
       const int t = min(strip0 + (p >> 5), tt.nstrips - 1) - strip0;
@@ -305,17 +326,24 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   // Group-wise int4 scale rows: chunk q = lane of row q / (BN/8) (lanes past
   // the rows repeat the last chunk into the unused tail of the region);
   // columns past N are clamped into the row (their outputs are not stored).
+  // A 128-wide block that ends 64 past K (KB = 2) repeats its last valid row.
   const _Float16* sbase = nullptr;
-  uint32_t soff = 0;
-  if (GS) {
-    const int gpb = a.gshift == 0 ? 2 : 1;  // scale rows per 64-wide K block
-    const int q = min(lane, gpb * (BN / 8) - 1);
-    const int r = q / (BN / 8), cc = q % (BN / 8);
+  uint32_t soff[GS ? S_LOADS : 1] = {}, soff_tail[GS && KB == 2 ? S_LOADS : 1] = {};
+  if constexpr (GS) {
+    const int gpb = KB == 2 ? 4 >> a.gshift : a.gshift == 0 ? 2 : 1;  // scale rows per stage
     const int n0 = strip0 * 16;
     sbase = tt.scale + n0;
-    soff = (uint32_t)(r * tt.N * 2 + min(n0 * 2 + cc * 16, tt.N * 2 - 16) - n0 * 2);
+#pragma unroll
+    for (int i = 0; i < S_LOADS; ++i) {
+      const int q = min(i * 64 + lane, gpb * (BN / 8) - 1);
+      const int r = q / (BN / 8), cc = q % (BN / 8);
+      const int col = min(n0 * 2 + cc * 16, tt.N * 2 - 16) - n0 * 2;
+      soff[i] = (uint32_t)(r * tt.N * 2 + col);
+      if constexpr (KB == 2)
+        soff_tail[i] = (uint32_t)(min(r, max((2 >> a.gshift) - 1, 0)) * tt.N * 2 + col);
+    }
   }
-  const bool k_tail = (a.K & 63) != 0;
+  const bool k_tail = (a.K & (64 * KB - 1)) != 0;
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8*)smem;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -341,21 +369,32 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
       // and are zeroed after they land (fix_tail).
 #pragma unroll
       for (int l = 0; l < A_LOADS; ++l) {
-        const uint32_t o = kb * 64 + acol[l] < a.K ? aoff[l] + kb * 128 : arow_off[l];
+        const uint32_t o = kb * 64 * KB + acol[l] < a.K ? aoff[l] + kb * 128 * KB : arow_off[l];
         dma16s(o, abase, st + (wave_u * A_LOADS + l) * 1024);
       }
     } else {
-      const uint8_t* ab = abase + kb * 128;
+      const uint8_t* ab = abase + kb * 128 * KB;
 #pragma unroll
       for (int l = 0; l < A_LOADS; ++l) dma16s(aoff[l], ab, st + (wave_u * A_LOADS + l) * 1024);
     }
-    const uint8_t* bb = bbase + (WF ? (int64_t)(kb >> 1) * kTileBytes + (kb & 1) * (kTileBytes / 2)
-                                    : (int64_t)kb * kTileBytes);
+    const uint8_t* bb = bbase + (WF && KB == 1
+                                     ? (int64_t)(kb >> 1) * kTileBytes + (kb & 1) * (kTileBytes / 2)
+                                     : (int64_t)kb * kTileBytes);
 #pragma unroll
     for (int l = 0; l < B_LOADS; ++l) dma16s(boff[l], bb, st + A_BYTES + (wave_u * B_LOADS + l) * 1024);
     (void)bb;
-    if (GS && wave_u == 0)
-      dma16s(soff, sbase + (int64_t)((2 * kb) >> a.gshift) * tt.N, st + S_OFF);
+    if constexpr (GS) {
+      if (wave_u == 0) {
+        const _Float16* sb = sbase + (int64_t)((2 * KB * kb) >> a.gshift) * tt.N;
+#pragma unroll
+        for (int l = 0; l < S_LOADS; ++l) {
+          uint32_t o = soff[l];
+          if constexpr (KB == 2)
+            if (may_tail && k_tail && kb == a.kblocks - 1) o = soff_tail[l];
+          dma16s(o, sb, st + S_OFF + l * 1024);
+        }
+      }
+    }
   };
   auto fix_tail = [&](int i) {  // local K block i (two K groups: zeroed by its group)
     const int kb = kb0 + i;
@@ -363,7 +402,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
     if constexpr (KG == 2) st = smem + ((i / KG) % STAGES) * STAGE + (i % KG) * SUB;
 #pragma unroll
     for (int l = 0; l < A_LOADS; ++l)
-      if (kb * 64 + acol[l] >= a.K)
+      if (kb * 64 * KB + acol[l] >= a.K)
         *reinterpret_cast<uint4*>(st + (wave * A_LOADS + l) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
   };
 
@@ -454,7 +493,39 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   auto compute = [&](int i) {
     const uint8_t* st = smem + (i % STAGES) * STAGE;
     if constexpr (KG == 2) st += kg_u * SUB;  // this wavefront's group's block
-    if constexpr (WF != kWfInt8 && IL) {
+    if constexpr (KB == 2) {
+      uint4 braw[TN];
+      _Float16 sc[GS ? TN : 1];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        braw[j] = *reinterpret_cast<const uint4*>(st + A_BYTES + (wn * TN + j) * kTileBytes + lane * 16);
+        // (this lane's 32 positions lie in one group: scale row g >> gshift)
+        if (GS)
+          sc[GS ? j : 0] = *reinterpret_cast<const _Float16*>(
+              st + S_OFF + (((lane >> 4) >> a.gshift) * BN + (wn * TN + j) * 16 + (lane & 15)) * 2);
+      }
+      const uint8_t* as = st + (lane >> 5) * A_SUB + arow * 128;
+      half8 af[4][TM];
+#pragma unroll
+      for (int step = 0; step < 4; ++step) {
+        const int ao = (a_chunk128(4 * ((lane >> 4) & 1) + step) ^ sw) * 16;
+#pragma unroll
+        for (int r = 0; r < TM; ++r)
+          af[step][r] = *reinterpret_cast<const half8*>(as + ao + r * 16 * 128);
+      }
+#pragma unroll
+      for (int step = 0; step < 4; ++step)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const uint32_t d = step == 0 ? braw[j].x : step == 1 ? braw[j].y : step == 2 ? braw[j].z : braw[j].w;
+          const half8 b = GS ? dequant8_i4_scaled(d, sc[GS ? j : 0]) : dequant8_i4(d);
+#pragma unroll
+          for (int r = 0; r < TM; ++r) acc[r][j] = mfma16x16x32(af[step][r], b, acc[r][j]);
+        }
+      // All LDS reads of the block go first (mask 0x100): one exposed LDS
+      // latency per block instead of one per MFMA step.
+      if constexpr (TM <= 4) __builtin_amdgcn_sched_group_barrier(0x100, (GS ? 2 : 1) * TN + 4 * TM, 0);
+    } else if constexpr (WF != kWfInt8 && IL) {
       // The int8 interleaved schedule below with int4 B (and group-wise
       // scale reads among the first LDS reads).
       __builtin_amdgcn_s_setprio(1);
@@ -599,7 +670,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < ns) issue(s, true);
-  // Group-wise int4: wavefront 0 issues one more DMA per K block (scale rows).
+  // Group-wise int4: wavefront 0 issues S_LOADS more DMAs per stage (scale rows).
   const bool extra = GS && wave_u == 0;
   // Steady state: the block issued (i + STAGES - 1 <= nk - 2) is never the
   // last one, so it holds no K tail, and STAGES - 2 blocks stay in flight
@@ -608,10 +679,10 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   int i = 0;
   for (; i < ns - STAGES; ++i) {
     if constexpr (STAGES - 2 >= 2) {
-      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (LOADS + 1)) : "memory");
+      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (LOADS + S_LOADS)) : "memory");
       else __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
     } else if constexpr (STAGES - 2 == 1) {
-      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + 1) : "memory");
+      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + S_LOADS) : "memory");
       else __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
     } else {
       __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -625,10 +696,10 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   for (; i < ns; ++i) {
     const int ahead = min(STAGES - 2, ns - 1 - i);  // stages issued after i
     if (ahead >= 2) {
-      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (LOADS + 1)) : "memory");
+      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (LOADS + S_LOADS)) : "memory");
       else __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
     } else if (ahead == 1) {
-      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + 1) : "memory");
+      if (extra) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + S_LOADS) : "memory");
       else __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
     } else {
       __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -728,7 +799,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
 // True when the 32-bit DMA offsets of w8a16_gemm_v3_kernel cannot overflow
 // for any projection of the launch.
 inline bool v3_offsets_fit(const GemmKernelArgs& ka, int bm, int bn) {
-  const uint64_t a_span = (uint64_t)bm * (uint64_t)ka.ldx * 2 + (uint64_t)ka.kblocks * 128;
+  const uint64_t a_span = (uint64_t)bm * (uint64_t)ka.ldx * 2 + (uint64_t)round_up(ka.K, kTileK4) * 2;
   const uint64_t b_span = (uint64_t)(bn / 16) * (uint64_t)ka.wtiles * kTileBytes;
   return a_span < (1ull << 32) && b_span < (1ull << 32);
 }
@@ -857,13 +928,13 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void w8a16_gemm_dma_kernel(
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int OCC, int WF = kWfInt8,
-          bool IL = false, bool BR = false, int KG = 1>
+          bool IL = false, bool BR = false, int KG = 1, int KB = 1>
 hipError_t launch_v3_t(const GemmKernelArgs& ka, hipStream_t stream) {
   const int64_t tiles = (int64_t)ka.tiles_m * ka.tiles_n;
   if (tiles <= 0 || tiles > 0x7fffffff || ka.splits < 1 || ka.splits > 65535 ||
       !v3_offsets_fit(ka, BM, BN))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL((w8a16_gemm_v3_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, OCC, WF, IL, BR, KG>),
+  hipLaunchKernelGGL((w8a16_gemm_v3_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, OCC, WF, IL, BR, KG, KB>),
                      dim3((unsigned)tiles, (unsigned)ka.splits), dim3(WAVES_M * WAVES_N * 64 * KG), 0,
                      stream, ka);
   return hipGetLastError();
@@ -899,15 +970,28 @@ enum GemmCfgId {
   kV3M64N64KG,    //   128x128 / 64x128 / 64x64 tiles (64x64: 4 stages)
   kV3M128N256KG,  // two K groups of the 128x256 register-B tile, 1 workgroup/CU: int8 long K
                   //   in about one round of tiles (plan_long_k_two_groups)
+  // int4 tiles of 128-wide K blocks (KB = 2), 4 wavefronts 1x4, 3 or 4 stages:
+  // M <= 64, and launches of few tiles beyond (plan_int4_small)
+  kI4M32N64,
+  kI4M32N128,
+  kI4M48N64,
+  kI4M48N128,
+  kI4M64N64,
+  kI4M64N128,
   kGemmCfgCount
 };
+
+// Configurations whose K blocks are 128 wide.
+constexpr bool gemm_cfg_k128(int cfg) { return cfg >= kI4M32N64 && cfg <= kI4M64N128; }
 
 // {BM, BN, workgroups per CU}
 constexpr int kGemmTile[kGemmCfgCount][3] = {{128, 256, 2}, {128, 128, 3}, {128, 128, 2},
                                              {64, 256, 2},  {128, 128, 1}, {32, 64, 4},
                                              {64, 64, 4},   {128, 128, 3}, {32, 128, 3},
                                              {32, 256, 2},  {128, 128, 1}, {64, 128, 1},
-                                             {64, 64, 1},   {128, 256, 1}};
+                                             {64, 64, 1},   {128, 256, 1},
+                                             {32, 64, 3},   {32, 128, 3},  {48, 64, 3},
+                                             {48, 128, 2},  {64, 64, 2},   {64, 128, 2}};
 
 // Wavefronts per workgroup of a configuration.
 int gemm_cfg_waves(int cfg) {
@@ -937,6 +1021,12 @@ const char* gemm_cfg_name(int cfg, int wf, int M) {
     case kV3M64N128KG: return "64x128 two K groups";
     case kV3M64N64KG: return "64x64 two K groups";
     case kV3M128N256KG: return "128x256 two K groups, B-in-registers";
+    case kI4M32N64: return "32x64 128-wide K blocks";
+    case kI4M32N128: return "32x128 128-wide K blocks";
+    case kI4M48N64: return "48x64 128-wide K blocks";
+    case kI4M48N128: return "48x128 128-wide K blocks";
+    case kI4M64N64: return "64x64 128-wide K blocks";
+    case kI4M64N128: return "64x128 128-wide K blocks";
     default: return "?";
   }
 }
@@ -958,6 +1048,12 @@ hipError_t launch_gemm4(int cfg, const GemmKernelArgs& ka, hipStream_t stream) {
       if (WF == kWfInt4Grp && ka.M >= 1024)
         return launch_v3_t<128, 128, 1, 4, 2, 3, WF, false, true>(ka, stream);
       return launch_v3_t<128, 128, 1, 4, 2, 3, WF, true>(ka, stream);
+    case kI4M32N64: return launch_v3_t<32, 64, 1, 4, 4, 3, WF, false, false, 1, 2>(ka, stream);
+    case kI4M32N128: return launch_v3_t<32, 128, 1, 4, 3, 3, WF, false, false, 1, 2>(ka, stream);
+    case kI4M48N64: return launch_v3_t<48, 64, 1, 4, 3, 3, WF, false, false, 1, 2>(ka, stream);
+    case kI4M48N128: return launch_v3_t<48, 128, 1, 4, 3, 2, WF, false, false, 1, 2>(ka, stream);
+    case kI4M64N64: return launch_v3_t<64, 64, 1, 4, 3, 2, WF, false, false, 1, 2>(ka, stream);
+    case kI4M64N128: return launch_v3_t<64, 128, 1, 4, 3, 2, WF, false, false, 1, 2>(ka, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -969,6 +1065,7 @@ constexpr int kMaxSplitTiles = kMaxSplitCounters;
 void set_tiles(GemmPlan& p, int M, const int* Ns, int nproj) {
   p.bm = kGemmTile[p.cfg][0];
   p.bn = kGemmTile[p.cfg][1];
+  p.span_rows = p.bm;
   p.tiles_m = (int)ceil_div(M, p.bm);
   p.tiles_n = 0;
   for (int i = 0; i < nproj; ++i) p.tiles_n += (int)ceil_div(Ns[i], p.bn);
@@ -1100,6 +1197,67 @@ static bool plan_long_k_two_groups(int M, const int* Ns, int nproj, int K, int c
   return false;
 }
 
+// Packed int4 at M <= 64 and on launches of few 128x128 tiles (t128) beyond:
+// the tiles of 128-wide K blocks.  These launches are bound by instruction
+// issue, not by memory (with every load aimed at cached lines they take the
+// same time): a stage is about 52 VALU operations per strip to dequantize plus
+// the MFMAs, and a CU with two workgroups does more of them per microsecond
+// than with one.  So the plan takes the least estimated time over the tiles
+// and 1..8 K splits of
+//   2.2 + 1.1 c + blocks * (c == 1 ? alone : c * shared) + hand-off us,
+// with c workgroups on the fullest CU, `blocks` 128-wide K blocks per
+// workgroup, the tile's time per block alone on a CU and when it shares one,
+// and a hand-off of 1.2 us + 0.4 us per split and 4096 outputs of the tile.
+// The constants are a least-squares fit to 5400 timed launches (MI355X, N
+// 512..37888, K 1024..25600, M 17..512, per-channel, gs 32 and 128; rms error
+// 8%); over those shapes its choice is 1.3..3% off the best one at M <= 128.
+// Against the plans before (the GEMV up to M 64, 64x256 and 128-row tiles
+// beyond): 0.61 of the time at M 33..64 (19456 x 2560 at M 48 28.9 -> 15.9
+// us, 5120 x 25600 68.3 -> 29.4), 0.70 at M 65..128 (1024 x 2048 at M 96 16.6
+// -> 7.2).  Beyond that the larger tiles reuse each dequantized weight for
+// more rows and win from half a tile per CU (5/4 up to M 128: one or two rows
+// of tiles); at K >= 8192 their K splits win from 64 tiles.
+static bool plan_int4_small(int M, const int* Ns, int nproj, int K, int cus, int64_t t128,
+                            GemmPlan& out) {
+  if (M > 128 && (2 * t128 > cus || (K >= 8192 && 4 * t128 >= cus))) return false;
+  if (M > 64 && 4 * t128 > 5LL * cus) return false;
+  struct Tile {
+    int cfg, max_m;
+    double alone, shared;  // us per 128-wide K block
+  };
+  constexpr Tile tiles[] = {
+      {kI4M32N64, 64, 0.343, 0.216},  {kI4M32N128, 64, 0.503, 0.368},
+      {kI4M48N64, 1 << 30, 0.415, 0.263}, {kI4M48N128, 1 << 30, 0.572, 0.449},
+      {kI4M64N64, 1 << 30, 0.500, 0.347}, {kI4M64N128, 1 << 30, 0.651, 0.532}};
+  const int kblocks = (int)ceil_div(K, kTileK4);
+  bool found = false;
+  double best = 0;
+  for (const Tile& t : tiles) {
+    GemmPlan p;
+    p.cfg = t.cfg;
+    set_tiles(p, M, Ns, nproj);
+    // Row strides are refused by the span of the larger tiles (64 rows below M
+    // 128, else 128), so which ones are does not depend on the tile taken here.
+    p.span_rows = M < 128 ? 64 : 128;
+    if (M > t.max_m || (p.bm > 32 && M <= p.bm - 16)) continue;  // rows of padding only
+    const int64_t n = (int64_t)p.tiles_m * p.tiles_n;
+    for (int s = 1; s <= kMaxGemmSplits; ++s) {
+      if (s > 1 && (kblocks < 4 * s || n > kMaxSplitTiles || n * s > 4LL * cus)) break;
+      p.kb_per_split = (int)ceil_div(kblocks, s);
+      p.splits = (int)ceil_div(kblocks, p.kb_per_split);
+      const double c = (double)ceil_div(n * p.splits, cus);
+      const double us = 2.2 + 1.1 * c + p.kb_per_split * (c == 1 ? t.alone : c * t.shared) +
+                        (p.splits > 1 ? 1.2 + 0.4 * p.splits * p.bm * p.bn / 4096 : 0.0);
+      if (!found || us < best) {
+        found = true;
+        best = us;
+        out = p;
+      }
+    }
+  }
+  return found;
+}
+
 GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev, bool int4) {
   const int cus = dev.cus > 0 ? dev.cus : 256;
   if (M <= 32 && !int4) {
@@ -1171,6 +1329,10 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
     GemmPlan kgp;
     if (plan_two_k_groups(M, Ns, nproj, K, cus, t128, kgp)) return kgp;
     if (plan_long_k_two_groups(M, Ns, nproj, K, cus, kgp)) return kgp;
+  }
+  if (int4) {
+    GemmPlan sp;
+    if (plan_int4_small(M, Ns, nproj, K, cus, t128, sp)) return sp;
   }
   GemmPlan p;
   if (M < 128) {
@@ -1263,9 +1425,10 @@ bool gemm_offsets_fit(const GemmPlan& p, int64_t ldx, int K, bool int4) {
   if (p.cfg == kDmaM128N128) return true;  // full per-lane addresses
   GemmKernelArgs ka;
   ka.ldx = ldx;
+  ka.K = K;
   ka.kblocks = (int)ceil_div(K, 64);
   ka.wtiles = int4 ? (int)ceil_div(K, kTileK4) : ka.kblocks;
-  return v3_offsets_fit(ka, p.bm, p.bn);
+  return v3_offsets_fit(ka, p.span_rows, p.bn);
 }
 
 // The v3 kernels address a tile with 32-bit offsets from its first row /
@@ -1301,7 +1464,7 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
   ka.ldx = pr.ldx;
   ka.M = pr.M;
   ka.K = pr.K;
-  ka.kblocks = (int)ceil_div(pr.K, 64);
+  ka.kblocks = (int)ceil_div(pr.K, gemm_cfg_k128(p.cfg) ? kTileK4 : 64);
   ka.wtiles = pr.wf ? (int)ceil_div(pr.K, kTileK4) : ka.kblocks;
   ka.gshift = pr.gshift;
   ka.nproj = pr.nproj;

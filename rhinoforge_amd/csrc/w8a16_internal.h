@@ -48,6 +48,7 @@ struct GemvPlan {
 struct GemmPlan {
   int cfg;       // tile configuration id (w8a16_gemm.hip)
   int bm, bn;    // workgroup tile
+  int span_rows; // rows of x the 32-bit offset check covers (>= bm)
   int tiles_m, tiles_n;  // tiles_n summed over the launch's projections
   int group_m;   // output-tile rows per scheduling group
   int splits;    // K splits across workgroups (1 = no workspace use)
@@ -79,7 +80,8 @@ bool gemm_offsets_fit(const GemmPlan& p, int64_t ldx, int K, bool int4);
 // not fit become the 64-bit-address kernel (unsplit); int4 plans unchanged.
 GemmPlan gemm_plan_for_stride(const GemmPlan& p, int M, const int* Ns, int nproj, int64_t ldx,
                               int K, bool int4);
-// int4: packed-int4 weights (TILE16X128_I4) take the large-tile rules only.
+// int4: packed-int4 weights (TILE16X128_I4) have tiles of their own at M <= 64
+// and on few-tile launches, and the large-tile rules beyond.
 GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev,
                    bool int4 = false);
 // GEMV plan of packed-int4 weights (nproj projections sharing x); grouped:
