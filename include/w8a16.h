@@ -108,6 +108,27 @@ int rf_w8a16_pack_weight_device(const int8_t* q_dev, int64_t N, int64_t K,
                                 int64_t ldq, void* dst_dev, size_t dst_bytes,
                                 void* stream);
 
+/* Floating weight types of rf_w8a16_quantize_device. */
+#define RF_W8A16_DTYPE_F16 0
+#define RF_W8A16_DTYPE_BF16 1
+#define RF_W8A16_DTYPE_F32 2
+
+/* Device quantizer, on `stream`: floating w[N,K] (row stride ldw elements) ->
+ * signed `bits`-wide values (8 or 4) and fp16 steps, with the arithmetic of
+ * the checkpoint converters (python/rpu_backend/quant/_common.py:10-36,
+ * quant/int4_pgrp_pack.py:33-60):
+ *   group_size 0        one step per row, from the row's largest fp16-rounded
+ *                       magnitude: scale[N]
+ *   32, 64, 128 (bits 4, K % group_size == 0)  one step per group of a row,
+ *                       from the fp32 values: scale[K / group_size][N]
+ *   layout ROWMAJOR     q int8 [N,K] row-major (N*K bytes)
+ *   layout TILE16X64    (bits 8, group_size 0) as rf_w8a16_pack_weight of those values
+ *   layout TILE16X128_I4 (bits 4) as rf_w4a16_pack_weight of those values
+ * scale is 2-byte, packed output 16-byte aligned; w aligned to its type. */
+int rf_w8a16_quantize_device(const void* w, int32_t dtype, int64_t N, int64_t K, int64_t ldw,
+                             int32_t bits, int32_t group_size, int32_t layout, void* q,
+                             size_t q_bytes, void* scale, void* stream);
+
 /* Kernel the AUTO policy runs for this shape on the current device
  * (RF_W8A16_KERNEL_GEMV or RF_W8A16_KERNEL_GEMM), or a negative status. */
 int rf_w8a16_select_kernel(int64_t M, int64_t N, int64_t K);

@@ -25,7 +25,7 @@ CSRC = PKG / "csrc"
 LIBDIR = PKG / "lib"
 INCLUDE = ROOT / "include"
 
-CAPI_SOURCES = ["w8a16_capi.hip", "w8a16_gemv.hip", "w8a16_gemm.hip"]
+CAPI_SOURCES = ["w8a16_capi.hip", "w8a16_gemv.hip", "w8a16_gemm.hip", "w8a16_quant.hip"]
 CAPI_LIB = LIBDIR / "librf_w8a16.so"
 TORCH_LIB = LIBDIR / "librf_w8a16_torch.so"
 BENCH_LIB = LIBDIR / "librf_bench.so"

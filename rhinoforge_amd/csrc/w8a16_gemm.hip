@@ -1208,7 +1208,7 @@ static bool plan_long_k_two_groups(int M, const int* Ns, int nproj, int K, int c
 // with c workgroups on the fullest CU, `blocks` 128-wide K blocks per
 // workgroup, the tile's time per block alone on a CU and when it shares one,
 // and a hand-off of 1.2 us + 0.4 us per split and 4096 outputs of the tile.
-// The constants are a least-squares fit to 5400 timed launches (MI355X, N
+// The constants are a least-squares fit to 11600 timed launches (MI355X, N
 // 512..37888, K 1024..25600, M 17..512, per-channel, gs 32 and 128; rms error
 // 8%); over those shapes its choice is 1.3..3% off the best one at M <= 128.
 // Against the plans before (the GEMV up to M 64, 64x256 and 128-row tiles

@@ -17,6 +17,9 @@
 //                Tensor?[] biases, int kernel=0) -> Tensor[]
 //   pack_weight(Tensor q) -> Tensor
 //   unpack_weight(Tensor packed, int N, int K) -> Tensor
+// and (namespace `rhinoforge`, what the Python quantizers run on a device):
+//   quantize(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)
+//   quantize_pack(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)
 //
 // These mirror the reference's eager FP16 `linear_into` (schema at
 // src/core/rpu_dispatch_registrations.inc:19-20, checks at
@@ -512,6 +515,77 @@ at::Tensor unpack_weight(const at::Tensor& packed, int64_t N, int64_t K) {
   return q;
 }
 
+// ---- Quantizers on the device ------------------------------------------------
+// Floating [N, K] weight -> values and fp16 steps (rf_w8a16_quantize_device),
+// row-major or packed.  The Python quantizers call these for plain HIP tensors
+// of a type the kernels read and keep their torch arithmetic for the rest.
+std::tuple<at::Tensor, at::Tensor> quantize_any(const at::Tensor& weight, int64_t bits,
+                                                int64_t group_size, int32_t layout,
+                                                const char* op) {
+  TORCH_CHECK(weight.dim() == 2 && weight.size(0) >= 1 && weight.size(1) >= 1, op,
+              ": weight must be a non-empty [N, K] matrix, got ", weight.sizes());
+  const at::ScalarType t = weight.scalar_type();
+  TORCH_CHECK(t == at::kHalf || t == at::kBFloat16 || t == at::kFloat, op,
+              ": weight must be float16, bfloat16 or float32, got ", t);
+  TORCH_CHECK(weight.is_cuda(), op, ": weight must be on a HIP device");
+  const int32_t dtype = t == at::kHalf ? RF_W8A16_DTYPE_F16
+                        : t == at::kBFloat16 ? RF_W8A16_DTYPE_BF16 : RF_W8A16_DTYPE_F32;
+  const int64_t N = weight.size(0), K = weight.size(1);
+  const at::Tensor w = (weight.stride(1) == 1 && weight.stride(0) >= K) ? weight : weight.contiguous();
+  const int64_t ldw = N == 1 ? std::max<int64_t>(K, w.stride(0)) : w.stride(0);
+  const auto opts = weight.options();
+  at::Tensor q;
+  if (layout == RF_W8A16_LAYOUT_ROWMAJOR) q = at::empty({N, K}, opts.dtype(at::kChar));
+  else if (layout == RF_W8A16_LAYOUT_TILE16X64) q = at::empty(packed_sizes_int8(N, K), opts.dtype(at::kChar));
+  else q = at::empty(packed_sizes_int4(N, K), opts.dtype(at::kByte));
+  TORCH_CHECK(group_size == 0 || K % group_size == 0, op, ": group_size=", group_size,
+              " does not divide K=", K);
+  at::Tensor s = group_size ? at::empty({K / group_size, N}, opts.dtype(at::kHalf))
+                            : at::empty({N}, opts.dtype(at::kHalf));
+  c10::DeviceGuard guard(weight.device());
+  void* stream = c10::hip::getCurrentHIPStream(weight.device().index()).stream();
+  check_status(rf_w8a16_quantize_device(w.data_ptr(), dtype, N, K, ldw, (int32_t)bits,
+                                        (int32_t)group_size, layout, q.data_ptr(),
+                                        (size_t)q.numel(), s.data_ptr(), stream),
+               op);
+  return {q, s};
+}
+
+// Values one int8 each, row-major [N, K]; steps [N] (group_size 0) or
+// [K / group_size, N].
+std::tuple<at::Tensor, at::Tensor> quantize(const at::Tensor& weight, int64_t bits,
+                                            int64_t group_size) {
+  return quantize_any(weight, bits, group_size, RF_W8A16_LAYOUT_ROWMAJOR, "rhinoforge::quantize");
+}
+
+// The same values packed: TILE16X64 tiles (8 bits) or TILE16X128_I4 tiles (4).
+std::tuple<at::Tensor, at::Tensor> quantize_pack(const at::Tensor& weight, int64_t bits,
+                                                 int64_t group_size) {
+  return quantize_any(weight, bits, group_size,
+                      bits == 8 ? RF_W8A16_LAYOUT_TILE16X64 : RF_W8A16_LAYOUT_TILE16X128_I4,
+                      "rhinoforge::quantize_pack");
+}
+
+at::Tensor quantize_steps_meta(const at::Tensor& weight, int64_t group_size) {
+  const auto o = weight.options().dtype(at::kHalf);
+  if (!group_size) return at::empty_symint({weight.sym_size(0)}, o);
+  return at::empty_symint({weight.sym_size(1) / group_size, weight.sym_size(0)}, o);
+}
+
+std::tuple<at::Tensor, at::Tensor> quantize_meta(const at::Tensor& weight, int64_t bits,
+                                                 int64_t group_size) {
+  return {at::empty_symint(weight.sym_sizes(), weight.options().dtype(at::kChar)),
+          quantize_steps_meta(weight, group_size)};
+}
+
+std::tuple<at::Tensor, at::Tensor> quantize_pack_meta(const at::Tensor& weight, int64_t bits,
+                                                      int64_t group_size) {
+  return {at::empty_symint({ceil_div(weight.sym_size(0), 16),
+                            ceil_div(weight.sym_size(1), bits == 8 ? 64 : 128), 1024},
+                           weight.options().dtype(bits == 8 ? at::kChar : at::kByte)),
+          quantize_steps_meta(weight, group_size)};
+}
+
 // ---- W4A16 -------------------------------------------------------------------
 // The reference's launcher takes a packed-int4 weight as a uint8 [N, K/2]
 // tensor and tells per-channel from group-wise by the scale's rank
@@ -855,5 +929,24 @@ TORCH_LIBRARY_IMPL(w4a16, CPU, m) {
 }
 TORCH_LIBRARY_IMPL(w4a16, Autograd, m) {
   for (const char* op : {"linear", "linear_multi", "pack_weight", "unpack_weight"})
+    m.impl(op, torch::CppFunction::makeFallthrough());
+}
+
+TORCH_LIBRARY(rhinoforge, m) {
+  m.def("quantize(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)");
+  m.def("quantize_pack(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)");
+}
+
+TORCH_LIBRARY_IMPL(rhinoforge, CUDA, m) {
+  m.impl("quantize", TORCH_FN(quantize));
+  m.impl("quantize_pack", TORCH_FN(quantize_pack));
+}
+TORCH_LIBRARY_IMPL(rhinoforge, Meta, m) {
+  m.impl("quantize", TORCH_FN(quantize_meta));
+  m.impl("quantize_pack", TORCH_FN(quantize_pack_meta));
+}
+// (callers pass detached weights: values and steps carry no graph)
+TORCH_LIBRARY_IMPL(rhinoforge, Autograd, m) {
+  for (const char* op : {"quantize", "quantize_pack"})
     m.impl(op, torch::CppFunction::makeFallthrough());
 }

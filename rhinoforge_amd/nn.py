@@ -33,6 +33,7 @@ from torch import nn
 
 from . import ops
 from .quant import quantize_linear_per_channel
+from .quant._common import on_kernel
 
 
 class _LogicalWeightStateDict:
@@ -155,7 +156,15 @@ class W8A16Linear(_LogicalWeightStateDict, nn.Module):
 
     @classmethod
     def from_linear(cls, linear: nn.Linear) -> "W8A16Linear":
-        """Quantize a floating nn.Linear per channel, then pack."""
+        """Quantize a floating nn.Linear per channel, then pack (on a HIP device
+        in one kernel, without the row-major values in between)."""
+        w = linear.weight.detach()
+        if on_kernel(w):
+            mod = cls(w.size(1), w.size(0), bias=linear.bias is not None, device="meta")
+            mod.weight, mod.weight_scale = torch.ops.rhinoforge.quantize_pack(w, 8, 0)
+            if linear.bias is not None:
+                mod.bias = linear.bias.detach().to(device=w.device, dtype=torch.float16).contiguous()
+            return mod
         q, s = quantize_linear_per_channel(linear.weight.detach())
         b = linear.bias.detach().to(torch.float16) if linear.bias is not None else None
         return cls.from_quantized(q, s, b)
@@ -256,6 +265,13 @@ class W4A16Linear(_LogicalWeightStateDict, nn.Module):
         reference's W4A16 converter, convert_qwen3_w4a16.py:40-42), then pack."""
         from .quant.int4 import quantize_int4_group_wise, quantize_int4_per_channel
         w = linear.weight.detach()
+        if group_size in (None, 0, 32, 64, 128) and on_kernel(w):
+            mod = cls(w.size(1), w.size(0), group_size=group_size or None,
+                      bias=linear.bias is not None, device="meta")
+            mod.weight, mod.weight_scale = torch.ops.rhinoforge.quantize_pack(w, 4, group_size or 0)
+            if linear.bias is not None:
+                mod.bias = linear.bias.detach().to(device=w.device, dtype=torch.float16).contiguous()
+            return mod
         if group_size:
             q, s, _ = quantize_int4_group_wise(w, group_size)
         else:

@@ -10,7 +10,8 @@ loads there and vice versa.  For a weight row ``w`` and ``L = 2**(bits-1)``:
     q     = clamp(rint(f32(w16) / f32(scale)), -L, L - 1)     ties to even
 
 Division and rounding are correctly rounded IEEE operations, so the CPU and a
-HIP device produce the same bytes.  The int4 quantizers in ``int4`` reuse the
+HIP device produce the same bytes.  On a HIP device the passes run as one
+kernel (``torch.ops.rhinoforge.quantize``) with the same arithmetic.  The int4 quantizers in ``int4`` reuse the
 scale and rounding steps below.
 """
 from __future__ import annotations
@@ -39,6 +40,20 @@ def round_to_levels(w32: torch.Tensor, step16: torch.Tensor, lo: int, hi: int) -
     return torch.round(w32 / step16.to(torch.float32)).clamp_(lo, hi).to(torch.int8)
 
 
+_KERNEL_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+
+
+def on_kernel(weight: torch.Tensor) -> bool:
+    """Whether the device quantizer takes this matrix: a plain HIP tensor (or
+    parameter) of a type it reads, non-empty, outside functorch transforms and
+    forward-mode AD.  Everything else keeps the torch arithmetic below, which
+    gives the same bytes."""
+    return (type(weight) in (torch.Tensor, torch.nn.Parameter) and weight.is_cuda
+            and weight.dim() == 2 and weight.dtype in _KERNEL_DTYPES and weight.numel() > 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 def _as_matrix(weight: torch.Tensor) -> torch.Tensor:
     if weight.dim() != 2:
         raise ValueError(f"a linear weight is a 2-D [out_features, in_features] matrix; "
@@ -54,6 +69,8 @@ def quantize_linear_per_channel(weight: torch.Tensor, *, bits: int = 8
     reference's fake-W4 checkpoint form); nothing is packed into nibbles.
     """
     lo, hi = signed_levels(bits)
+    if on_kernel(weight):
+        return torch.ops.rhinoforge.quantize(weight.detach(), bits, 0)
     w32 = _as_matrix(weight).to(torch.float16).to(torch.float32)
     step = scale_from_amax(w32.abs().amax(dim=1), hi)
     return round_to_levels(w32, step.unsqueeze(1), lo, hi), step
