@@ -129,6 +129,15 @@ int rf_w8a16_quantize_device(const void* w, int32_t dtype, int64_t N, int64_t K,
                              int32_t bits, int32_t group_size, int32_t layout, void* q,
                              size_t q_bytes, void* scale, void* stream);
 
+/* Int8 embedding lookup, on `stream`: y[m][h] = fp16(f32(table[id][h]) *
+ * f32(scale[id])) for id = ids[m] (python/rpu_backend/adapters/qwen3.py:654-680).
+ *   table : int8 [V,H] row-major;  scale : fp16 [V];  y : fp16 [M,H]
+ *   ids   : int64 (ids64 != 0) or int32 [M], in [-V, V) (negative ids count
+ *           from the end); an id outside aborts the kernel, so the stream's
+ *           next synchronization reports an error. */
+int rf_w8a16_embedding(const void* table, int64_t V, int64_t H, const void* scale,
+                       const void* ids, int32_t ids64, int64_t M, void* y, void* stream);
+
 /* Kernel the AUTO policy runs for this shape on the current device
  * (RF_W8A16_KERNEL_GEMV or RF_W8A16_KERNEL_GEMM), or a negative status. */
 int rf_w8a16_select_kernel(int64_t M, int64_t N, int64_t K);

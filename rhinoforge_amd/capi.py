@@ -86,6 +86,9 @@ SIGNATURES = {
     "rf_w8a16_quantize_device": (_c.c_int, [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int64,
                                             _c.c_int64, _c.c_int32, _c.c_int32, _c.c_int32,
                                             _c.c_void_p, _c.c_size_t, _c.c_void_p, _c.c_void_p]),
+    "rf_w8a16_embedding": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_int64, _c.c_void_p,
+                                      _c.c_void_p, _c.c_int32, _c.c_int64, _c.c_void_p,
+                                      _c.c_void_p]),
     "rf_w4a16_packed_bytes": (_c.c_size_t, [_c.c_int64, _c.c_int64]),
     "rf_w4a16_pack_weight": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64,
                                         _c.c_void_p, _c.c_size_t]),

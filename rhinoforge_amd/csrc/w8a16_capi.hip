@@ -396,6 +396,16 @@ int rf_w8a16_quantize_device(const void* w, int32_t dtype, int64_t N, int64_t K,
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
 }
 
+int rf_w8a16_embedding(const void* table, int64_t V, int64_t H, const void* scale,
+                       const void* ids, int32_t ids64, int64_t M, void* y, void* stream) {
+  if (check_nk(V, H) != RF_W8A16_OK || M < 1 || M > kMaxDim || !table || !scale || !ids || !y)
+    return RF_W8A16_EINVAL;
+  if (!aligned(scale, 2) || !aligned(y, 2) || !aligned(ids, ids64 ? 8 : 4)) return RF_W8A16_EALIGN;
+  const hipError_t e = rf::launch_embed(static_cast<const int8_t*>(table), V, H, scale, ids,
+                                        ids64 != 0, M, y, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
+}
+
 int rf_w8a16_select_kernel(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || M > kMaxDim || check_nk(N, K) != RF_W8A16_OK) return -RF_W8A16_EINVAL;
   return auto_kernel(M, N, K);

@@ -122,6 +122,8 @@ hipError_t launch_pack4(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint
                         hipStream_t stream);
 hipError_t launch_quantize(const void* w, int dtype, int64_t N, int64_t K, int64_t ldw, int bits,
                            int group, int layout, void* q, void* scale, hipStream_t stream);
+hipError_t launch_embed(const int8_t* table, int64_t V, int64_t H, const void* scale,
+                        const void* ids, bool ids64, int64_t M, void* y, hipStream_t stream);
 hipError_t launch_pack(const int8_t* q, int64_t N, int64_t K, int64_t ldq,
                        uint8_t* dst, hipStream_t stream);
 

@@ -1,6 +1,7 @@
-// Load-time quantizers (gfx950): floating weights -> quantized values,
-// row-major or already in the compute kernels' tile order.  Bound by memory:
-// one read of the input, one write of the output.
+// Load-time quantizers and the int8 embedding gather (gfx950): floating
+// weights -> quantized values, row-major or already in the compute kernels'
+// tile order; table rows -> fp16.  Bound by memory: one read of the input, one
+// write of the output.
 //
 // Quantizer arithmetic (the steps of rhinoforge_amd/quant/_common.py and
 // int4.py, bit for bit):
@@ -256,6 +257,48 @@ __global__ __launch_bounds__(256) void quant_groups_kernel(QuantArgs a) {
   store_chunk<LAYOUT>(a, n, c, qv);
 }
 
+// Row gather of an int8 table: y[m][h] = fp16(f32(q[id][h]) * f32(s[id])), the
+// product exact in fp32 and rounded once.  One workgroup per 256 * VEC outputs
+// of a row; VEC int8 values per thread (16-byte loads, 32-byte stores).
+template <int VEC, typename Id>
+__global__ __launch_bounds__(256) void embed_kernel(const int8_t* __restrict__ table, int64_t V,
+                                                    int64_t H, const _Float16* __restrict__ scale,
+                                                    const Id* __restrict__ ids, int per_row,
+                                                    _Float16* __restrict__ y) {
+  const int64_t m = blockIdx.x / (uint32_t)per_row;
+  const int64_t h = ((int64_t)(blockIdx.x - (uint32_t)m * (uint32_t)per_row) * 256 + threadIdx.x) * VEC;
+  int64_t id = (int64_t)ids[m];
+  if (id < 0) id += V;  // as torch indexing counts from the end
+  if ((uint64_t)id >= (uint64_t)V) __builtin_trap();  // an index out of range is an error
+  if (h >= H) return;
+  const float s = (float)scale[id];
+  const int8_t* q = table + id * H + h;
+  _Float16* o = y + m * H + h;
+  if constexpr (VEC == 1) {
+    *o = (_Float16)((float)*q * s);
+  } else {
+    uint32_t d[VEC / 4];
+    if constexpr (VEC == 16) {
+      const uint4 t = load_u4(q);
+      d[0] = t.x; d[1] = t.y; d[2] = t.z; d[3] = t.w;
+    } else {
+      const uint2 t = *reinterpret_cast<const uint2*>(q);
+      d[0] = t.x; d[1] = t.y;
+    }
+    uint32_t r[VEC / 2];
+#pragma unroll
+    for (int i = 0; i < VEC / 2; ++i) {
+      const int b = 2 * i;
+      const float f0 = (float)(int8_t)(d[b >> 2] >> (8 * (b & 3))) * s;
+      const float f1 = (float)(int8_t)(d[b >> 2] >> (8 * (b & 3) + 8)) * s;
+      r[i] = __builtin_bit_cast(uint32_t, half2v{(_Float16)f0, (_Float16)f1});
+    }
+#pragma unroll
+    for (int i = 0; i < VEC / 8; ++i)
+      reinterpret_cast<uint4*>(o)[i] = make_uint4(r[4 * i], r[4 * i + 1], r[4 * i + 2], r[4 * i + 3]);
+  }
+}
+
 template <int DT>
 hipError_t launch_quant_t(const QuantArgs& a, int layout, hipStream_t stream) {
   const dim3 block(256);
@@ -282,6 +325,21 @@ hipError_t launch_quant_t(const QuantArgs& a, int layout, hipStream_t stream) {
     default:
       hipLaunchKernelGGL((quant_rows_kernel<DT, RF_W8A16_LAYOUT_TILE16X128_I4>), grid, block, 0, stream, a);
   }
+  return hipGetLastError();
+}
+
+template <int VEC>
+hipError_t launch_embed_t(const int8_t* table, int64_t V, int64_t H, const _Float16* scale,
+                          const void* ids, bool ids64, int64_t M, _Float16* y, hipStream_t stream) {
+  const int64_t per_row = ceil_div(H, 256 * VEC);
+  if (M * per_row > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(M * per_row));
+  if (ids64)
+    hipLaunchKernelGGL((embed_kernel<VEC, int64_t>), grid, dim3(256), 0, stream, table, V, H, scale,
+                       static_cast<const int64_t*>(ids), (int)per_row, y);
+  else
+    hipLaunchKernelGGL((embed_kernel<VEC, int32_t>), grid, dim3(256), 0, stream, table, V, H, scale,
+                       static_cast<const int32_t*>(ids), (int)per_row, y);
   return hipGetLastError();
 }
 
@@ -316,6 +374,17 @@ hipError_t launch_quantize(const void* w, int dtype, int64_t N, int64_t K, int64
     case kDtBf16: return launch_quant_t<kDtBf16>(a, layout, stream);
     default: return launch_quant_t<kDtF32>(a, layout, stream);
   }
+}
+
+hipError_t launch_embed(const int8_t* table, int64_t V, int64_t H, const void* scale,
+                        const void* ids, bool ids64, int64_t M, void* y, hipStream_t stream) {
+  const _Float16* s = static_cast<const _Float16*>(scale);
+  _Float16* o = static_cast<_Float16*>(y);
+  if (H % 16 == 0 && aligned_to(table, 16) && aligned_to(y, 16))
+    return launch_embed_t<16>(table, V, H, s, ids, ids64, M, o, stream);
+  if (H % 8 == 0 && aligned_to(table, 8) && aligned_to(y, 16))
+    return launch_embed_t<8>(table, V, H, s, ids, ids64, M, o, stream);
+  return launch_embed_t<1>(table, V, H, s, ids, ids64, M, o, stream);
 }
 
 }  // namespace rf

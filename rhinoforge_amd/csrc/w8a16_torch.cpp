@@ -17,7 +17,8 @@
 //                Tensor?[] biases, int kernel=0) -> Tensor[]
 //   pack_weight(Tensor q) -> Tensor
 //   unpack_weight(Tensor packed, int N, int K) -> Tensor
-// and (namespace `rhinoforge`, what the Python quantizers run on a device):
+// and (namespace `rhinoforge`, what the Python quantizers and W8A16Embedding run):
+//   embedding(Tensor weight, Tensor weight_scale, Tensor ids) -> Tensor
 //   quantize(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)
 //   quantize_pack(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)
 //
@@ -839,6 +840,64 @@ at::Tensor w4_unpack_weight(const at::Tensor& packed, int64_t N, int64_t K) {
   return q;
 }
 
+// ---- Int8 embedding ------------------------------------------------------------
+// The lookup in torch operations: CPU tensors, and whatever the kernel does not
+// take (mask ids, another scale type, a layout of its own, autograd).
+at::Tensor embedding_eager(const at::Tensor& weight, const at::Tensor& scale,
+                           const at::Tensor& ids) {
+  const c10::List<c10::optional<at::Tensor>> idx({c10::optional<at::Tensor>(ids)});
+  const at::Tensor rows = at::index(weight, idx).to(at::kFloat);
+  return (rows * at::index(scale, idx).to(at::kFloat).unsqueeze(-1)).to(at::kHalf);
+}
+
+bool int_ids(const at::Tensor& ids) {
+  return ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt;
+}
+
+at::Tensor embedding_hip(const at::Tensor& weight, const at::Tensor& scale, const at::Tensor& ids) {
+  RECORD_FUNCTION("rhinoforge::embedding", {});
+  const bool kernel = int_ids(ids) && weight.scalar_type() == at::kChar && weight.dim() == 2 &&
+                      scale.scalar_type() == at::kHalf && scale.dim() == 1 &&
+                      scale.size(0) == weight.size(0) && weight.is_contiguous() &&
+                      scale.is_contiguous() && weight.numel() > 0 && ids.numel() > 0 &&
+                      ids.device() == weight.device() && scale.device() == weight.device() &&
+                      // (the launch grid: one workgroup per 256 values at the narrowest)
+                      ids.numel() * ceil_div(weight.size(1), 256) <= 0x7fffffff;
+  if (!kernel) return embedding_eager(weight, scale, ids);
+  const int64_t V = weight.size(0), H = weight.size(1), M = ids.numel();
+  const at::Tensor i = ids.contiguous();
+  std::vector<int64_t> shape = ids.sizes().vec();
+  shape.push_back(H);
+  at::Tensor y = at::empty(shape, weight.options().dtype(at::kHalf));
+  c10::DeviceGuard dev_guard(weight.device());
+  void* stream = c10::hip::getCurrentHIPStream(weight.device().index()).stream();
+  check_status(rf_w8a16_embedding(weight.data_ptr(), V, H, scale.data_ptr(), i.data_ptr(),
+                                  i.scalar_type() == at::kLong, M, y.data_ptr(), stream),
+               "rhinoforge::embedding");
+  return y;
+}
+
+at::Tensor embedding_meta(const at::Tensor& weight, const at::Tensor& scale,
+                          const at::Tensor& ids) {
+  if (!int_ids(ids) || weight.dim() != 2) return embedding_eager(weight, scale, ids);
+  std::vector<c10::SymInt> shape = ids.sym_sizes().vec();
+  shape.push_back(weight.sym_size(1));
+  return at::empty_symint(shape, weight.options().dtype(at::kHalf));
+}
+
+// Gradients (and forward-mode tangents) of the scale go through the torch form;
+// without any the kernel runs.
+at::Tensor embedding_autograd(const at::Tensor& weight, const at::Tensor& scale,
+                              const at::Tensor& ids) {
+  if ((at::GradMode::is_enabled() && scale.requires_grad()) || scale._fw_grad(0).defined())
+    return embedding_eager(weight, scale, ids);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("rhinoforge::embedding", "")
+                             .typed<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&)>();
+  return op.call(weight, scale, ids);
+}
+
 int64_t select_kernel(int64_t M, int64_t N, int64_t K) {
   const int k = rf_w8a16_select_kernel(M, N, K);
   TORCH_CHECK(k > 0, "w8a16::select_kernel: ", rf_w8a16_status_str(-k));
@@ -935,13 +994,18 @@ TORCH_LIBRARY_IMPL(w4a16, Autograd, m) {
 TORCH_LIBRARY(rhinoforge, m) {
   m.def("quantize(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)");
   m.def("quantize_pack(Tensor weight, int bits, int group_size) -> (Tensor, Tensor)");
+  m.def("embedding(Tensor weight, Tensor weight_scale, Tensor ids) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(rhinoforge, CUDA, m) {
   m.impl("quantize", TORCH_FN(quantize));
   m.impl("quantize_pack", TORCH_FN(quantize_pack));
+  m.impl("embedding", TORCH_FN(embedding_hip));
 }
+TORCH_LIBRARY_IMPL(rhinoforge, CPU, m) { m.impl("embedding", TORCH_FN(embedding_eager)); }
+TORCH_LIBRARY_IMPL(rhinoforge, FuncTorchBatched, m) { m.impl("embedding", TORCH_FN(embedding_eager)); }
 TORCH_LIBRARY_IMPL(rhinoforge, Meta, m) {
+  m.impl("embedding", TORCH_FN(embedding_meta));
   m.impl("quantize", TORCH_FN(quantize_meta));
   m.impl("quantize_pack", TORCH_FN(quantize_pack_meta));
 }
@@ -949,4 +1013,5 @@ TORCH_LIBRARY_IMPL(rhinoforge, Meta, m) {
 TORCH_LIBRARY_IMPL(rhinoforge, Autograd, m) {
   for (const char* op : {"quantize", "quantize_pack"})
     m.impl(op, torch::CppFunction::makeFallthrough());
+  m.impl("embedding", TORCH_FN(embedding_autograd));
 }

@@ -308,8 +308,8 @@ class W8A16Embedding(nn.Module):
     The checkpoint form of ``quantized_embed_tokens`` (quant/load.py:303-316,
     343-356): ``weight`` int8 [V, H], ``weight_scale`` fp16 [V].  A lookup
     gathers rows and dequantizes them as ``fp16(f32(q) * f32(s))``
-    (adapters/qwen3.py:654-680); the table is gathered, never multiplied, so
-    it stays row-major.
+    (adapters/qwen3.py:654-680), in one kernel on a HIP device; the table is
+    gathered, never multiplied, so it stays row-major.
     """
 
     def __init__(self, weight: torch.Tensor, weight_scale: torch.Tensor,
@@ -327,9 +327,7 @@ class W8A16Embedding(nn.Module):
         self.register_buffer("weight_scale", weight_scale.contiguous())
 
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
-        rows = self.weight[input_ids].to(torch.float32)
-        return (rows * self.weight_scale[input_ids].to(torch.float32).unsqueeze(-1)
-                ).to(torch.float16)
+        return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
 
     def extra_repr(self) -> str:
         return f"{self.num_embeddings}, {self.embedding_dim}, int8 rows"

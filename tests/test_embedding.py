@@ -1,0 +1,77 @@
+"""W8A16Embedding's lookup op: every index form that torch indexing takes, on
+the CPU and under meta / vmap / autograd, against the torch expression; the HIP
+kernel (16-, 8- and 1-wide) byte for byte against the same on the GPU."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import rhinoforge_amd as rf
+
+
+def _table(v, h, dev="cpu"):
+    g = torch.Generator().manual_seed(v + h)
+    q = torch.randint(-128, 128, (v, h), generator=g, dtype=torch.int8)
+    s = (torch.rand(v, generator=g) * 0.01).half()
+    s[0] = 6e-8                                    # fp16 subnormal products
+    return q.to(dev), s.to(dev)
+
+
+def _want(q, s, ids):
+    return (q[ids].float() * s[ids].float().unsqueeze(-1)).half()
+
+
+def _forms(v, dev):
+    base = torch.tensor([[0, 1, v - 1], [-1, -v, v // 2]], device=dev)
+    mask = torch.zeros(v, dtype=torch.bool, device=dev)
+    mask[::3] = True
+    return {"int64": base, "int32": base.int(), "transposed": base.t(), "scalar": base[0, 1],
+            "empty": base[:0], "mask": mask, "one row": base[0, :1]}
+
+
+def _check(q, s, dev):
+    emb = rf.W8A16Embedding(q, s)
+    for name, ids in _forms(q.size(0), dev).items():
+        got, want = emb(ids), _want(q, s, ids)
+        assert got.shape == want.shape and got.dtype == torch.float16, name
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), name
+
+
+def test_cpu_forms():
+    q, s = _table(50, 24)
+    _check(q, s, "cpu")
+    with pytest.raises(IndexError):
+        rf.W8A16Embedding(q, s)(torch.tensor([50]))
+    with pytest.raises(IndexError):
+        rf.W8A16Embedding(q, s)(torch.tensor([0.5]))
+
+
+def test_transforms():
+    q, s = _table(50, 24)
+    ids = torch.tensor([[3, 1], [-1, 7]])
+    emb = rf.W8A16Embedding(q, s)
+    assert torch.equal(torch.vmap(emb)(ids), _want(q, s, ids))
+    sg = s.clone().requires_grad_()
+    emb.weight_scale = sg
+    emb(ids).float().sum().backward()
+    ref = s.clone().requires_grad_()
+    _want(q, ref, ids).float().sum().backward()
+    assert torch.equal(sg.grad, ref.grad)
+    m = torch.ops.rhinoforge.embedding(q.to("meta"), s.to("meta"), ids.to("meta"))
+    assert m.shape == (2, 2, 24) and m.dtype == torch.float16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("v,h", [(300, 4096), (97, 4112), (50, 24), (33, 8), (20, 7), (9, 1),
+                                 (1000, 5120)])
+def test_gpu_forms(v, h):
+    print(f"embedding {v}x{h}", flush=True)
+    q, s = _table(v, h, "cuda")
+    _check(q, s, "cuda")
+    wide = torch.zeros(v * h + 3, dtype=torch.int8, device="cuda")   # a misaligned table
+    odd = wide[3:].view(v, h).copy_(q)
+    ids = torch.randint(-v, v, (3, 70), device="cuda")
+    emb = rf.W8A16Embedding(odd, s)
+    assert torch.equal(emb(ids), _want(q, s, ids))
+    strided = torch.as_strided(ids, (35, 3), (2, 70))
+    assert torch.equal(emb(strided), _want(q, s, strided))
