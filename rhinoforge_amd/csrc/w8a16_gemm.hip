@@ -1132,11 +1132,22 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
   // two K splits and >= 0.75 workgroups per CU.
   const bool beyond = M > 512;
   if (beyond && kblocks > 80) return false;
-  // At M 33..64 only the 64x64 form with four K splits over <= 64 tiles
+  // At M 33..64 on <= 64 tiles of 64x64 only that form with four K splits
   // (K >= 4096): -8..-14% against the 64x64 4-stage tile with 8 splits at
-  // N 1024..4096, K 4096..8192; at N 5120 / 8192 mixed (-7..+4%).
+  // N 1024..4096, K 4096..8192; at N 5120 / 8192 mixed (-7..+4%).  From 96
+  // tiles (N >= 6144 in all) and K 2048 on, the 64x128 and 64x64 forms by the
+  // estimate below: one round of workgroups that each fill a CU, where 64x64
+  // tiles with four to eight splits left CUs with one or two more than others
+  // (M 41: Qwen3-VL-32B q/k/v, three splits of 64x128, 17.9 instead of 21.3
+  // us; 19456 x 2560 17.7 instead of 21.8; 12288 x 2048 11.6 instead of 13.7).
   const bool one_row = M <= 64;
-  if (one_row && kblocks < 64) return false;
+  bool many = false;
+  if (one_row) {
+    int64_t t64 = 0;
+    for (int i = 0; i < nproj; ++i) t64 += ceil_div(Ns[i], 64);
+    many = 8 * t64 >= 3LL * cus && kblocks >= 32;
+    if (!many && kblocks < 64) return false;
+  }
   struct Cand {
     int cfg;
     double rate;  // TFLOP/s per CU
@@ -1149,8 +1160,11 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
     p.cfg = c.cfg;
     set_tiles(p, M, Ns, nproj);
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    if (one_row && (c.cfg != kV3M64N64KG || 4 * tiles > cus)) continue;
-    for (int s = 1; s <= 4; s *= 2) {
+    if (one_row && (many ? c.cfg == kV3M128N128KG
+                         : c.cfg != kV3M64N64KG || 4 * tiles > cus)) continue;
+    for (int s = 1; s <= 4; ++s) {
+      // (three splits only where four of the 128-wide forms do not fit one round)
+      if (s == 3 && (c.cfg == kV3M64N64KG || 4 * tiles <= cus)) continue;
       if (tiles * s > cus || kblocks < 16 * s || (s > 1 && tiles > kMaxSplitTiles)) continue;
       if (beyond && (s > 2 || 4 * tiles * s < 3LL * cus)) continue;
       const int kbs = (int)ceil_div(kblocks, s);
@@ -1297,7 +1311,11 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
     // Qwen3-8B gate/up at M 48..64: 28.5 instead of 30.5..32 us; MI355X).
     int64_t w256 = 0;
     for (int i = 0; i < nproj; ++i) w256 += ceil_div(Ns[i], 256);
-    const bool wide = w256 * 4 >= 3LL * cus;
+    // With two splits that make more than one round of workgroups, some CUs
+    // get two and set the pace: there one unsplit tile per workgroup is ahead
+    // although it leaves CUs idle (37888 x 3584 at M 41, 148 tiles: 36.0
+    // instead of 47.2 us; 34816 x 5120, 136 tiles: 47.9 instead of 60.0).
+    const bool wide = w256 * 4 >= 3LL * cus || w256 * 2 > cus;
     if (wide || (w256 * 8 >= 3LL * cus && kblocks >= 2 * kMinKbPerSplit)) {
       p.cfg = kV3M64N256;
       set_tiles(p, M, Ns, nproj);
@@ -1307,6 +1325,20 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
     }
     GemmPlan kgp;
     if (plan_two_k_groups(M, Ns, nproj, K, cus, /*t128=*/0, kgp)) return kgp;
+    if (kblocks >= 256) {
+      // Long K on more than 64 tiles: as many splits of the 64x128 form (up
+      // to six) as fit one round (5120 x 25600 at M 41 33.7 instead of 40.5
+      // us, at M 64 35.6 instead of 45.8 with eight splits of 64x64).
+      p.cfg = kV3M64N128KG;
+      set_tiles(p, M, Ns, nproj);
+      const int64_t n = (int64_t)p.tiles_m * p.tiles_n;
+      const int s = (int)(cus / n < 6 ? cus / n : 6);
+      if (s >= 3 && n <= kMaxSplitTiles) {
+        p.kb_per_split = (int)ceil_div(kblocks, s);
+        p.splits = (int)ceil_div(kblocks, p.kb_per_split);
+        return p;
+      }
+    }
     p.cfg = kV3M64N64;
     set_tiles(p, M, Ns, nproj);
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
