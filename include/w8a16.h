@@ -150,7 +150,9 @@ typedef struct rf_w8a16_plan_info {
   int32_t kernel;           /* RF_W8A16_KERNEL_GEMV or RF_W8A16_KERNEL_GEMM */
   int32_t tile_m;           /* activation rows per workgroup (GEMV: 16 per m-tile) */
   int32_t tile_n;           /* output channels per workgroup, per projection */
-  int32_t splits;           /* K splits across workgroups (1: no workspace use) */
+  int32_t splits;           /* K splits across workgroups (1: no workspace use); of the
+                               last tiles only where workgroups < tiles * splits: those
+                               run unsplit if the workspace lacks workspace_bytes */
   int32_t waves;            /* wavefronts per workgroup */
   int32_t workgroups;       /* workgroups of the launch, all splits */
   uint64_t workspace_bytes; /* workspace the launch uses past the counter region */

@@ -477,6 +477,10 @@ int rf_w8a16_plan(int64_t M, const int64_t* Ns, int32_t count, int64_t K, int32_
     out->splits = p.splits;
     out->waves = rf::gemm_cfg_waves(p.cfg);
     out->workgroups = p.tiles_m * p.tiles_n * p.splits;
+    if (p.rem_splits > 1) {
+      out->splits = p.rem_splits;
+      out->workgroups = p.rem0 + (p.tiles_m * p.tiles_n - p.rem0) * p.rem_splits;
+    }
     out->workspace_bytes = rf::gemm_workspace_bytes(p);
     snprintf(out->name, sizeof(out->name), "gemm %s", rf::gemm_cfg_name(p.cfg, format, (int)M));
   }
@@ -586,9 +590,11 @@ static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
       return too_small;
     e = rf::launch_gemv(pr, p, p.splits > 1 ? workspace : nullptr, s);
   } else {
-    const rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev);
-    if (p.splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) return too_small;
-    e = rf::launch_gemm(pr, p, p.splits > 1 ? workspace : nullptr, s);
+    rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev);
+    // (the split of the last tiles is left out where its scratch is missing)
+    if (p.rem_splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
+    if (const size_t extra = rf::gemm_workspace_bytes(p); extra && !workspace_ok(extra)) return too_small;
+    e = rf::launch_gemm(pr, p, rf::gemm_workspace_bytes(p) ? workspace : nullptr, s);
   }
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
 }
@@ -774,11 +780,12 @@ int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs
       return RF_W8A16_EWORKSPACE;
     e = rf::launch_gemv(pr, p, p.splits > 1 ? workspace : nullptr, s);
   } else {
-    const rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev, true);
+    rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev, true);
+    if (p.rem_splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
     // The int4 GEMM has no 64-bit-address kernel.
     if (!rf::gemm_offsets_fit(p, ldx, pr.K, true)) return RF_W8A16_EKERNEL;
-    if (p.splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) return RF_W8A16_EWORKSPACE;
-    e = rf::launch_gemm(pr, p, p.splits > 1 ? workspace : nullptr, s);
+    if (const size_t extra = rf::gemm_workspace_bytes(p); extra && !workspace_ok(extra)) return RF_W8A16_EWORKSPACE;
+    e = rf::launch_gemm(pr, p, rf::gemm_workspace_bytes(p) ? workspace : nullptr, s);
   }
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
 }

@@ -64,8 +64,11 @@ struct GemmKernelArgs {
   GemmProj proj[kMaxProj];
   int splits;            // K splits (blockIdx.y); 1 = no workspace
   int kb_per_split;
-  float* partial;        // [splits][tiles][BM*BN], fp32
-  uint32_t* counters;    // [tiles], zero between calls
+  // Tiles from rem0 on run in rem_splits K splits of rem_kb blocks each, the
+  // ones before it unsplit (rem_splits > 1 only with splits == 1).
+  int rem0, rem_splits, rem_kb;
+  float* partial;        // [splits][split tiles][BM*BN], fp32
+  uint32_t* counters;    // [split tiles], zero between calls
   int wtiles;            // 1 KB weight tiles per strip along K (64 positions int8, 128 int4)
   int gshift;            // group-wise int4: log2(group_size / 32)
 };
@@ -283,15 +286,26 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
   const int wave = KG == 1 ? (tid >> 6) : (tid >> 6) % NW;
   const int kg_u = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / NW);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int tile = blockIdx.x;
-  const int split = blockIdx.y;
+  int tile = blockIdx.x;
+  int split = blockIdx.y;
+  int splits = a.splits, kb_split = a.kb_per_split;
+  int ptile = tile, ptiles = a.tiles_m * a.tiles_n;  // this tile among the split ones
+  if (a.rem_splits > 1 && tile >= a.rem0) {
+    ptiles -= a.rem0;
+    ptile -= a.rem0;
+    split = ptile / ptiles;
+    ptile -= split * ptiles;
+    tile = a.rem0 + ptile;
+    splits = a.rem_splits;
+    kb_split = a.rem_kb;
+  }
   int tile_m, tile_n;
   tile_of(tile, a, tile_m, tile_n);
   const TileTarget tt = target_of(a, tile_n);
   const int m0 = tile_m * BM;
   const int strip0 = tt.tn * B_TILES;
-  const int kb0 = split * a.kb_per_split;
-  const int nk = min(a.kblocks - kb0, a.kb_per_split);  // K blocks of this split (>= 1)
+  const int kb0 = split * kb_split;
+  const int nk = min(a.kblocks - kb0, kb_split);  // K blocks of this split (>= 1)
 
   // Wave-uniform bases and per-lane 32-bit offsets.
   const uint8_t* abase = reinterpret_cast<const uint8_t*>(a.x + (int64_t)m0 * a.ldx);
@@ -737,15 +751,14 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
     }
   }
 
-  if (a.splits > 1) {
+  if (splits > 1) {
     // Partial tile in lane order: element (wave, i, j, r) of lane l at
     // ((((wave*TM + i)*TN + j)*4 + r)*64 + l) floats, so every store and
     // load below moves 256 contiguous bytes per wavefront.
     constexpr uint32_t TILE_F = BM * BN;
-    const int tiles = a.tiles_m * a.tiles_n;
     const __amdgpu_buffer_rsrc_t pr =
-        partial_rsrc(a.partial, (uint32_t)((uint64_t)a.splits * tiles * TILE_F * 4));
-    const uint32_t own = ((uint32_t)split * tiles + tile) * TILE_F * 4;
+        partial_rsrc(a.partial, (uint32_t)((uint64_t)splits * ptiles * TILE_F * 4));
+    const uint32_t own = ((uint32_t)split * ptiles + ptile) * TILE_F * 4;
     if (kg_u == 0) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -766,15 +779,15 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
     barrier_lds();
     if (tid == 0) {
       const uint32_t prev =
-          __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      is_last = prev == (uint32_t)(a.splits - 1) ? 1u : 0u;
+          __hip_atomic_fetch_add(&a.counters[ptile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      is_last = prev == (uint32_t)(splits - 1) ? 1u : 0u;
     }
     barrier_lds();
     if (!is_last) return;
     // Last to arrive: sum every split's partial (its own included, read
     // back) in split order, so the result does not depend on arrival order.
-    for (int sp = 0; sp < a.splits && kg_u == 0; ++sp) {
-      const uint32_t base = ((uint32_t)sp * tiles + tile) * TILE_F * 4;
+    for (int sp = 0; sp < splits && kg_u == 0; ++sp) {
+      const uint32_t base = ((uint32_t)sp * ptiles + ptile) * TILE_F * 4;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -788,7 +801,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
           }
     }
     if (tid == 0)
-      __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&a.counters[ptile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
   if (kg_u != 0) return;  // group 0 holds the tile's sums
@@ -934,8 +947,10 @@ hipError_t launch_v3_t(const GemmKernelArgs& ka, hipStream_t stream) {
   if (tiles <= 0 || tiles > 0x7fffffff || ka.splits < 1 || ka.splits > 65535 ||
       !v3_offsets_fit(ka, BM, BN))
     return hipErrorInvalidValue;
+  const int64_t gx = ka.rem_splits > 1 ? ka.rem0 + (tiles - ka.rem0) * ka.rem_splits : tiles;
+  if (gx > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((w8a16_gemm_v3_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, OCC, WF, IL, BR, KG, KB>),
-                     dim3((unsigned)tiles, (unsigned)ka.splits), dim3(WAVES_M * WAVES_N * 64 * KG), 0,
+                     dim3((unsigned)gx, (unsigned)ka.splits), dim3(WAVES_M * WAVES_N * 64 * KG), 0,
                      stream, ka);
   return hipGetLastError();
 }
@@ -943,7 +958,8 @@ hipError_t launch_v3_t(const GemmKernelArgs& ka, hipStream_t stream) {
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES>
 hipError_t launch_dma_t(const GemmKernelArgs& ka, hipStream_t stream) {
   const int64_t tiles = (int64_t)ka.tiles_m * ka.tiles_n;
-  if (tiles <= 0 || tiles > 0x7fffffff || ka.splits != 1) return hipErrorInvalidValue;
+  if (tiles <= 0 || tiles > 0x7fffffff || ka.splits != 1 || ka.rem_splits > 1)
+    return hipErrorInvalidValue;
   hipLaunchKernelGGL((w8a16_gemm_dma_kernel<BM, BN, WAVES_M, WAVES_N, STAGES>),
                      dim3((unsigned)tiles), dim3(WAVES_M * WAVES_N * 64), 0, stream, ka);
   return hipGetLastError();
@@ -1450,6 +1466,27 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
   if ((p.cfg == kV3M128N128 || p.cfg == kV3M128N128S3) && p.splits == 1 && tiles > cus &&
       tiles <= 2LL * cus)
     p.cfg = kV3M128N128IL;
+  // 128x256 tiles in whole rounds of CUs and a few (up to a quarter round)
+  // more: the CUs that get one of those set the pace (800 tiles are 3.125 per
+  // CU and take nearly four).  The K range of the last tiles is split into
+  // fewer pieces than CUs, so that they give most CUs one more, smaller, piece
+  // of work (at least 3/4 of the CUs, at least eight K blocks each).  MI355X,
+  // graph-timed, rotated weights: 51200 x 5120 at M 512 (800 tiles, seven
+  // pieces each of the last 32) 244 -> 217 us, 34816 x 5120 at M 1000 (1088,
+  // 64 in three) 294 -> 266, int4 322 -> 279; 24576 x 4096 at M 1300 (1056) 233
+  // -> 210.  128x128 tiles (three per CU) gain nothing or lose (7168 x 5120 at
+  // M 640, 280 tiles, +9%): their CUs already overlap three tiles.
+  const int64_t rem = tiles % cus;
+  if (p.cfg == kV3M128N256 && p.splits == 1 && tiles > cus && rem > 0 && 4 * rem <= cus &&
+      kblocks >= 48) {
+    int s2 = (int)((cus - 1) / rem < kMaxGemmSplits ? (cus - 1) / rem : kMaxGemmSplits);
+    while (s2 > 1 && kblocks < 8 * s2) --s2;
+    if (s2 > 1 && 4 * rem * s2 >= 3LL * cus) {
+      p.rem0 = (int)(tiles - rem);
+      p.rem_kb = (int)ceil_div(kblocks, s2);
+      p.rem_splits = (int)ceil_div(kblocks, p.rem_kb);
+    }
+  }
   return p;
 }
 
@@ -1474,14 +1511,16 @@ GemmPlan gemm_plan_for_stride(const GemmPlan& plan, int M, const int* Ns, int np
   p.cfg = kDmaM128N128;
   set_tiles(p, M, Ns, nproj);
   p.splits = 1;
+  p.rem_splits = 1;
   p.kb_per_split = (int)ceil_div(K, 64);
   return p;
 }
 
 size_t gemm_workspace_bytes(const GemmPlan& p) {
-  if (p.splits <= 1) return 0;
-  return (size_t)p.splits * (size_t)p.tiles_m * (size_t)p.tiles_n * (size_t)p.bm * (size_t)p.bn *
-         sizeof(float);
+  const size_t tiles = (size_t)p.tiles_m * (size_t)p.tiles_n;
+  const size_t parts = p.splits > 1 ? (size_t)p.splits * tiles
+                       : p.rem_splits > 1 ? (size_t)p.rem_splits * (tiles - (size_t)p.rem0) : 0;
+  return parts * (size_t)p.bm * (size_t)p.bn * sizeof(float);
 }
 
 hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* workspace,
@@ -1525,9 +1564,12 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
     }
     ka.splits = q.splits;
     ka.kb_per_split = q.kb_per_split;
+    ka.rem0 = q.rem0;
+    ka.rem_splits = q.rem_splits;
+    ka.rem_kb = q.rem_kb;
     ka.partial = nullptr;
     ka.counters = nullptr;
-    if (q.splits > 1) {
+    if (q.splits > 1 || q.rem_splits > 1) {
       ka.counters = static_cast<uint32_t*>(workspace);
       ka.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + RF_W8A16_WS_COUNTER_BYTES);
     }
@@ -1539,7 +1581,7 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
     p = gemm_plan_for_stride(p, pr.M, ns, pr.nproj, pr.ldx, pr.K, false);
   }
   fill(p);
-  if (p.splits > 1 && (!workspace || (int64_t)p.tiles_m * p.tiles_n > kMaxSplitTiles ||
+  if ((p.splits > 1 || p.rem_splits > 1) && (!workspace || (int64_t)p.tiles_m * p.tiles_n > kMaxSplitTiles ||
                        gemm_workspace_bytes(p) >= (1ull << 31)))
     return hipErrorInvalidValue;
   if (pr.wf == kWfInt4) return launch_gemm4<kWfInt4>(p.cfg, ka, stream);

@@ -53,6 +53,9 @@ struct GemmPlan {
   int group_m;   // output-tile rows per scheduling group
   int splits;    // K splits across workgroups (1 = no workspace use)
   int kb_per_split;
+  // With splits == 1: tiles from rem0 on in rem_splits K splits of rem_kb
+  // blocks (1: none).
+  int rem0 = 0, rem_splits = 1, rem_kb = 0;
 };
 
 struct DeviceInfo {

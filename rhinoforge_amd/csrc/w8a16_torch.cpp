@@ -108,10 +108,14 @@ WorkspaceCache& workspace_cache() {
 // refuses a workspace that is too small with RF_W8A16_EWORKSPACE before it
 // launches anything; only then is the size the shape needs queried (a second
 // launch plan), the buffer grown and the call repeated.
+// From M rows on where the GEMM may split the K range of its last tiles only if
+// there is room (it runs them whole otherwise), the size is queried up front.
+constexpr int64_t kQueryRows = 129;
 template <typename Call, typename Need>
-int with_workspace(const at::Device& dev, void* stream, const char* op, Call call, Need need) {
+int with_workspace(const at::Device& dev, void* stream, int64_t M, const char* op, Call call,
+                   Need need) {
   WorkspaceCache& wc = workspace_cache();
-  at::Tensor ws = wc.get(dev, stream, 0);
+  at::Tensor ws = wc.get(dev, stream, M >= kQueryRows ? need() : 0);
   int st = call(ws.data_ptr(), (size_t)ws.numel());
   if (st == RF_W8A16_EWORKSPACE) {
     const size_t bytes = need();
@@ -226,7 +230,7 @@ void launch(const Checked& c, const at::Tensor& weight, const at::Tensor& scale,
   void* stream = c10::hip::getCurrentHIPStream(c.x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const int st = with_workspace(
-      c.x2.device(), stream, op,
+      c.x2.device(), stream, c.M, op,
       [&](void* ws, size_t ws_bytes) {
         return rf_w8a16_linear(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(), (int32_t)layout,
                                scale.data_ptr(), bptr, y.data_ptr(), c.N, c.M, c.N, c.K,
@@ -304,7 +308,7 @@ std::vector<at::Tensor> linear_multi_hip(const at::Tensor& input, at::TensorList
     c10::DeviceGuard guard(c0.x2.device());
     void* stream = c10::hip::getCurrentHIPStream(c0.x2.device().index()).stream();
     const int st = with_workspace(
-        c0.x2.device(), stream, op,
+        c0.x2.device(), stream, c0.M, op,
         [&](void* ws, size_t ws_bytes) {
           return rf_w8a16_linear_multi(c0.x2.data_ptr(), c0.x2.stride(0), (int32_t)layout, projs,
                                        (int32_t)count, c0.M, c0.K, (int32_t)kernel, ws, ws_bytes,
@@ -459,7 +463,7 @@ std::tuple<at::Tensor, at::Tensor> linear_argmax_hip(const at::Tensor& input,
   void* stream = c10::hip::getCurrentHIPStream(c.x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const int st = with_workspace(
-      c.x2.device(), stream, op,
+      c.x2.device(), stream, c.M, op,
       [&](void* ws, size_t ws_bytes) {
         return rf_w8a16_linear_argmax(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(),
                                       (int32_t)layout, scale.data_ptr(), bptr,
@@ -670,7 +674,7 @@ at::Tensor w4_linear_hip(const at::Tensor& input, const at::Tensor& weight, cons
   void* stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const int st = with_workspace(
-      x2.device(), stream, op,
+      x2.device(), stream, M, op,
       [&](void* ws, size_t ws_bytes) {
         return rf_w4a16_linear(x2.data_ptr(), x2.stride(0), weight.data_ptr(), sc.data_ptr(),
                                (int32_t)group_size, bptr, y.data_ptr(), N, M, N, K,
@@ -757,7 +761,7 @@ std::vector<at::Tensor> w4_linear_multi_hip(const at::Tensor& input, at::TensorL
   c10::DeviceGuard dev_guard(x2.device());
   void* stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
   const int st = with_workspace(
-      x2.device(), stream, op,
+      x2.device(), stream, M, op,
       [&](void* ws, size_t ws_bytes) {
         return rf_w4a16_linear_multi(x2.data_ptr(), x2.stride(0), projs, (int32_t)count,
                                      (int32_t)group_size, M, K, (int32_t)kernel, ws, ws_bytes,

@@ -27,6 +27,14 @@ ROWS = [
     (100, [5112], 4104, "gemm 64x128 two K groups", 3),
 ]
 
+# 128x256 tiles in whole rounds of CUs and a few more, whose K range is split:
+# (M, N per projection, K, tiles past the whole rounds, pieces of each)
+LAST_TILES = [
+    (500, [12800, 38300], 3080, 32, 6),   # 4 x 200 tiles, ragged N, K tail in the last piece
+    (1000, [17400, 17408], 4104, 64, 3),  # 8 x 136 tiles, ragged M
+    (1300, [24576], 3072, 32, 6),
+]
+
 
 def _id(r):
     return f"{r[0]}x{'_'.join(map(str, r[1]))}x{r[2]}"
@@ -60,3 +68,56 @@ def test_parity(row):
         rep = o.check_tolerance(y.cpu().numpy()[rows], o.cpu_path(x[rows], q, s),
                                 o.oracle_fp64(x[rows], q, s))
         assert rep.ok, str(rep)
+
+
+@pytest.mark.parametrize("row", LAST_TILES, ids=_id)
+def test_last_tiles_plan(row):
+    m, ns, k, rem, pieces = row
+    tiles = -(-m // 128) * sum(-(-n // 256) for n in ns)
+    assert tiles % 256 == rem
+    for fmt in (0, 1, 2):
+        if fmt and (k % 64 or any(n % 16 for n in ns)):
+            continue
+        p = capi.plan(m, ns, k, fmt=fmt, cus=256)
+        assert (p["name"], p["splits"]) == ("gemm 128x256 B-in-registers", pieces), p
+        assert p["workgroups"] == tiles - rem + rem * pieces
+        assert p["workspace_bytes"] == rem * pieces * 128 * 256 * 4
+        assert p["workspace_bytes"] + capi.WS_COUNTER_BYTES <= capi.NOALLOC_SCRATCH_BYTES
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row", LAST_TILES, ids=_id)
+def test_last_tiles_parity(row):
+    """Split last tiles, also without the workspace they need (run whole): both
+    within the bar, the first bit-identical on a second call."""
+    import ctypes
+    m, ns, k = row[:3]
+    print(f"last tiles M={m} N={ns} K={k}", flush=True)
+    x = o.make_activation(o.derive_seed(78, "x", m, k), m, k)
+    g = torch.Generator().manual_seed(k)
+    qs = [torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8) for n in ns]
+    ss = [(torch.rand(n, generator=g) * 1e-3 + 1e-4).half() for n in ns]
+    xd = torch.from_numpy(x).cuda()
+    ws = [rf.pack_weight(q.cuda()) for q in qs]
+    sd = [s.cuda() for s in ss]
+    ys = rf.linear_multi(xd, ws, sd)
+    again = rf.linear_multi(xd, ws, sd)
+    lib = capi.load()
+    bare = [torch.empty_like(y) for y in ys]
+    projs = (capi.Proj * len(ns))()
+    for i, n in enumerate(ns):
+        projs[i] = capi.Proj(ws[i].data_ptr(), sd[i].data_ptr(), None, bare[i].data_ptr(), n, n)
+    st = lib.rf_w8a16_linear_multi(xd.data_ptr(), k, 1, projs, len(ns), m, k, 0, None, 0,
+                                   ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert st == capi.OK, capi.status_str(st)
+    rows = np.unique(np.r_[0:2, m // 2, 127, 128, m - 2:m])
+    tiles_n = [-(-n // 256) for n in ns]
+    for q, s, y, y2, y3, n, t in zip(qs, ss, ys, again, bare, ns, tiles_n):
+        assert torch.equal(y, y2)
+        cols = np.r_[0:40, (t - 1) * 256: n]     # the first and the last tile column
+        for out in (y, y3):
+            rep = o.check_tolerance(out.cpu().numpy()[rows][:, cols],
+                                    o.cpu_path(x[rows], q.numpy()[cols], s.numpy()[cols]),
+                                    o.oracle_fp64(x[rows], q.numpy()[cols], s.numpy()[cols]))
+            assert rep.ok, str(rep)
