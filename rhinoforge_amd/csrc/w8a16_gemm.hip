@@ -122,29 +122,6 @@ __device__ __forceinline__ void tile_of(int bid, const GemmKernelArgs& a, int& t
   tn = r / gm;
 }
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// dma16 (w8a16_common.h) with a wave-uniform SGPR base and a per-lane
-// 32-bit byte offset (global_load_lds_dwordx4 voff, s[base]).
-__device__ __forceinline__ void dma16s(uint32_t voff, const void* sbase, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// Chunk swizzle of the LDS A tile: 16-byte chunk c of row r is stored in
-// slot c ^ a_swizzle(r).  An MFMA A-fragment read has 16 lanes on rows
-// r0..r0+15 (r0 % 16 == 0) at one chunk, and the next 16 lanes on the same
-// rows at chunk ^ 2; with this swizzle the accesses of every 8-, 16- and
-// 32-lane group cover distinct LDS banks (64 or 128 banks of 4 bytes).
-__device__ __forceinline__ int a_swizzle(int r) { return (r & 7) ^ (((r >> 3) & 1) * 5); }
-
-// 128-wide K blocks: there the second 16 lanes of a fragment read are at
-// chunk ^ 4, so chunks are stored with bits 1 and 2 of their index exchanged
-// (its own inverse), which makes that slot ^ 2 again.  (A read of the plain
-// order runs at half the rate: 290 against 494 GB/s per CU, eight wavefronts.)
-__device__ __forceinline__ int a_chunk128(int c) { return (c & 1) | ((c & 2) << 1) | ((c & 4) >> 1); }
-
 // Buffer resource over the split-K partials; accesses use sc1 (device-scope
 // coherent: written through / re-fetched past the issuing XCD's L2, the
 // same instructions as relaxed agent-scope atomic stores and loads).
