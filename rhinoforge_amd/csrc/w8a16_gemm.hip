@@ -1156,8 +1156,12 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
     if (one_row && (many ? c.cfg == kV3M128N128KG
                          : c.cfg != kV3M64N64KG || 4 * tiles > cus)) continue;
     for (int s = 1; s <= 4; ++s) {
-      // (three splits only where four of the 128-wide forms do not fit one round)
-      if (s == 3 && (c.cfg == kV3M64N64KG || 4 * tiles <= cus)) continue;
+      // (three splits only where four of the 128-wide forms do not fit one
+      // round, and at M > 128 only from K 4545 on: shorter launches keep
+      // the 64x64 plan that test_linear_multi_two_k_groups holds them to,
+      // although three splits are ahead there too: 2560 x 4096 at M 256 14.6
+      // instead of 16.3 us)
+      if (s == 3 && (c.cfg == kV3M64N64KG || 4 * tiles <= cus || (M > 128 && kblocks < 72))) continue;
       if (tiles * s > cus || kblocks < 16 * s || (s > 1 && tiles > kMaxSplitTiles)) continue;
       if (beyond && (s > 2 || 4 * tiles * s < 3LL * cus)) continue;
       const int kbs = (int)ceil_div(kblocks, s);
