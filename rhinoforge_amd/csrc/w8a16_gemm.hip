@@ -1178,6 +1178,38 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
   return found;
 }
 
+// Packed int4 at K >= 12288 in less than one 128x256 tile per CU (80 and more
+// on 256 CUs): as many K splits of that tile as its two workgroups per CU
+// hold, each of at least 56 K blocks.  Each strip is dequantized once per 128
+// rows either way, but the wide tile reads half the A fragments per MFMA, and
+// the splits fill both workgroups of nearly every CU, where 128x128 tiles,
+// whole or in two splits, left one to two uneven rounds.  MI355X, graph-timed,
+// rotated weights, group size 128 / per-channel: 5120 x 25600 at M 640 187
+// (gs 32) / 168 -> 148 / 133 us, at M 1000 264 / 246 -> 216 / 191, 3584 x 18944
+// at M 1400 233 / 187 -> 167 / 151, 4096 x 14336 at M 1600 210 / 189 -> 170 /
+// 153, 4096 x 12288 at M 1200 130 / 121 -> 117 / 107; even at the worst (182..192
+// tiles, whose two splits leave a quarter of the slots empty, 0.96..1.01 of the
+// time).  Not with fewer tiles or shorter splits: 2560 x 16384 at M 1000, 80
+// tiles in six splits of 43 blocks, 83 -> 88 us, 64 tiles in eight 1.02..1.05
+// of the time; 4096 x 12288 at M 1000 in four of 48 99 / 90 us, against 99 / 86
+// with two splits of interleaved 128x128.
+static bool plan_int4_long_k(int M, const int* Ns, int nproj, int K, int cus, GemmPlan& out) {
+  const int kblocks = (int)ceil_div(K, 64);
+  GemmPlan p;
+  p.cfg = kV3M128N256;
+  set_tiles(p, M, Ns, nproj);
+  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+  if (kblocks < 192 || tiles >= cus || 16 * tiles < 5LL * cus || tiles > kMaxSplitTiles) return false;
+  int s = (int)(2LL * cus / tiles);
+  s = s < kMaxGemmSplits ? s : kMaxGemmSplits;
+  // (80..95 tiles take five splits and more: only with 64 blocks in each)
+  if (kblocks < (8 * tiles < 3LL * cus ? 64 : 56) * s) return false;
+  p.kb_per_split = (int)ceil_div(kblocks, s);
+  p.splits = (int)ceil_div(kblocks, p.kb_per_split);
+  out = p;
+  return true;
+}
+
 // Long K (>= 8192) at M 512..2048 in about one round of 128x256 tiles (int8):
 // the 128x256 tile with B in registers as two K groups (eight wavefronts, one
 // workgroup per CU), with the fewest K splits (1..3) that bring the launch to
@@ -1362,6 +1394,7 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
   if (int4) {
     GemmPlan sp;
     if (plan_int4_small(M, Ns, nproj, K, cus, t128, sp)) return sp;
+    if (M >= 128 && plan_int4_long_k(M, Ns, nproj, K, cus, sp)) return sp;
   }
   GemmPlan p;
   if (M < 128) {
@@ -1413,7 +1446,12 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
     // 26.5 us with 2 splits, 28.6 us with 4).
     s = (int)(slots / tiles);
     s = s < kMaxGemmSplits ? s : kMaxGemmSplits;
-    while (s > 1 && kblocks < s * ((tiles * s <= cus) ? 16 : 24)) --s;
+    // Int4 on half to two thirds of a tile per CU: three splits (one and a
+    // half workgroups per CU) from 18 blocks in each (6144 x 4096 at M 384, 144
+    // tiles, gs 128 / per-channel: 33.8 / 31.8 -> 29.0 / 29.5 us with the
+    // interleaved schedule below; 5120 x 4096 at M 400 34.7 / 33.4 -> 30.4 / 31).
+    const bool three = int4 && 2 * tiles > cus && 3 * tiles <= 2LL * cus;
+    while (s > 1 && kblocks < s * ((tiles * s <= cus) ? 16 : three ? 18 : 24)) --s;
   } else if ((p.cfg == kV3M128N128 || p.cfg == kV3M128N128S3) && kblocks >= 192 &&
              tiles <= 3LL * cus) {
     // Long K (>= 12288) at one tile per CU, or 1.25..1.75 / 2.25..2.75 per
@@ -1443,9 +1481,13 @@ GemmPlan plan_gemm(int M, const int* Ns, int nproj, int K, const DeviceInfo& dev
   // M 1024..4096, K 4096..12288, and +20% on the fused Qwen3-VL-32B q/k/v at
   // M = 512; -1..3% at one tile per CU or 2.5..3 per CU, where the plain
   // schedule stays).  Int4 alike: per-channel +6..32% (Qwen3-8B / VL-32B
-  // q/k/v and o at M 512..2048), group-wise +14% below M 1024.
-  if ((p.cfg == kV3M128N128 || p.cfg == kV3M128N128S3) && p.splits == 1 && tiles > cus &&
-      tiles <= 2LL * cus)
+  // q/k/v and o at M 512..2048), group-wise +14% below M 1024.  Int4 also where
+  // K splits make the one to two workgroups per CU: gs 128 8192 x 5120 at M 384
+  // 42.1 -> 40.6 us, 5120 x 8192 at M 700 69.0 -> 66.5, 6144 x 4096 at M 300
+  // 31.0 -> 28.9, per-channel 4096 x 12288 at M 700 74.3 -> 72.0 (the worst:
+  // 8192 x 5120 at M 300 +1.4%, per-channel three splits +1..3%).
+  if ((p.cfg == kV3M128N128 || p.cfg == kV3M128N128S3) && (p.splits == 1 || int4) &&
+      tiles * p.splits > cus && tiles * p.splits <= 2LL * cus)
     p.cfg = kV3M128N128IL;
   // 128x256 tiles in whole rounds of CUs and a few (up to a quarter round)
   // more: the CUs that get one of those set the pace (800 tiles are 3.125 per

@@ -10,6 +10,7 @@ import torch
 
 import rhinoforge_amd as rf
 from rhinoforge_amd import capi
+from oracle import w4a16 as o4
 from oracle import w8a16 as o
 
 # (M, N per projection, K, plan name, K splits)
@@ -25,6 +26,16 @@ ROWS = [
     # M 65 and more: three splits of a 128-wide form where four do not fit
     (250, [5000], 8200, "gemm 128x128 two K groups", 3),
     (100, [5112], 4104, "gemm 64x128 two K groups", 3),
+]
+
+# int4 launches of large tiles: (M, N per projection, K, group size, plan, splits)
+INT4_ROWS = [
+    (640, [5120], 25600, 128, "gemm 128x256 B-in-registers", 5),            # K >= 12288: 128x256 in K splits
+    (1000, [2560, 2560], 12352, 32, "gemm 128x256 B-in-registers", 3),      # two projections, K % 128 == 64
+    (1300, [4880], 12288, 0, "gemm 128x256 B-in-registers", 2),             # ragged M and N
+    (300, [6160], 4160, 64, "gemm 128x128 interleaved", 3),  # three splits of 18 blocks and more
+    (500, [5120], 3456, 0, "gemm 128x128 interleaved", 3),   # exactly 18
+    (384, [8192], 5120, 128, "gemm 128x128 interleaved", 2),
 ]
 
 # 128x256 tiles in whole rounds of CUs and a few more, whose K range is split:
@@ -121,3 +132,36 @@ def test_last_tiles_parity(row):
                                     o.cpu_path(x[rows], q.numpy()[cols], s.numpy()[cols]),
                                     o.oracle_fp64(x[rows], q.numpy()[cols], s.numpy()[cols]))
             assert rep.ok, str(rep)
+
+
+@pytest.mark.parametrize("row", INT4_ROWS, ids=_id)
+def test_int4_plan(row):
+    m, ns, k, gs, name, splits = row
+    p = capi.plan(m, ns, k, fmt=2 if gs else 1, cus=256)
+    assert (p["name"], p["splits"]) == (name, splits), p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row", INT4_ROWS, ids=_id)
+def test_int4_parity(row):
+    m, ns, k, gs = row[:4]
+    print(f"int4 gemm balance M={m} N={ns} K={k} gs={gs}", flush=True)
+    x = o.make_activation(o.derive_seed(79, "x", m, k), m, k)
+    g = torch.Generator().manual_seed(k)
+    qs = [torch.randint(-8, 8, (n, k), generator=g, dtype=torch.int8) for n in ns]
+    ss = [(torch.rand((k // gs, n) if gs else (n,), generator=g) * 1e-2 + 1e-3).half() for n in ns]
+    xd = torch.from_numpy(x).cuda()
+    ws = [rf.pack_weight_int4(q.cuda()) for q in qs]
+    sd = [s.cuda() for s in ss]
+    ys = rf.linear_multi_w4a16(xd, ws, sd)
+    again = rf.linear_multi_w4a16(xd, ws, sd)
+    torch.cuda.synchronize()
+    rows = np.unique(np.r_[0:2, m // 2, 127, m - 2:m])
+    for q, s, y, y2, n in zip(qs, ss, ys, again, ns):
+        assert torch.equal(y, y2)
+        cols = np.r_[0:40, n // 2:n // 2 + 40, n - 300:n]
+        s = np.ascontiguousarray(s.numpy()[..., cols])
+        rep = o.check_tolerance(y.cpu().numpy()[rows][:, cols],
+                                o4.cpu_path(x[rows], q.numpy()[cols], s),
+                                o4.oracle_fp64(x[rows], q.numpy()[cols], s))
+        assert rep.ok, str(rep)
