@@ -947,7 +947,7 @@ hipError_t launch_dma_t(const GemmKernelArgs& ka, hipStream_t stream) {
 // Tile configurations (measured on MI355X over the BASELINE prefill shapes).
 enum GemmCfgId {
   kV3M128N256,    // 4 wavefronts 1x4, 2 stages, 2 workgroups/CU, B in registers: wide launches,
-                  // and every launch beyond six 128x128 tiles per CU
+                  // every launch beyond six 128x128 tiles per CU, int4 long K in K splits
   kV3M128N128,    // 4 wavefronts 1x4, 2 stages, 3 workgroups/CU, B in registers: M >= 1024 up to
                   // six 128x128 tiles per CU, and K-split launches above one workgroup per CU
   kV3M128N128S3,  // 4 wavefronts 1x4, 3 stages, 2 workgroups/CU: 128 <= M < 1024, N < 16384
@@ -955,7 +955,7 @@ enum GemmCfgId {
   kDmaM128N128,   // 64-bit addresses: when the v3 32-bit offsets could overflow
   kV3M32N64,      // 4 wavefronts 1x4, 3 stages, 4 workgroups/CU: M <= 32, with K splits
   kV3M64N64,      // 4 wavefronts 1x4, 4 stages, 4 workgroups/CU: M 33..64, with K splits
-  kV3M128N128IL,  // kV3M128N128 with the interleaved MFMA schedule: 1..2 tiles per CU
+  kV3M128N128IL,  // kV3M128N128 with the interleaved MFMA schedule: 1..2 workgroups per CU
   kV3M32N128,     // 4 wavefronts 1x4, 4 stages, 3 workgroups/CU: M <= 32, >= 0.75 tiles per CU
   kV3M32N256,     // 4 wavefronts 1x4, 3 stages, 2 workgroups/CU: M <= 32, >= 0.75 tiles per CU
   kV3M128N128KG,  // two K groups of 4 wavefronts, 3 stages, 1 workgroup/CU: int8 M 33..2048,
