@@ -1604,8 +1604,10 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
     p = gemm_plan_for_stride(p, pr.M, ns, pr.nproj, pr.ldx, pr.K, false);
   }
   fill(p);
-  if ((p.splits > 1 || p.rem_splits > 1) && (!workspace || (int64_t)p.tiles_m * p.tiles_n > kMaxSplitTiles ||
-                       gemm_workspace_bytes(p) >= (1ull << 31)))
+  // (of a launch that splits its last tiles only those have counters)
+  const int64_t split_tiles = (int64_t)p.tiles_m * p.tiles_n - (p.rem_splits > 1 ? p.rem0 : 0);
+  if ((p.splits > 1 || p.rem_splits > 1) &&
+      (!workspace || split_tiles > kMaxSplitTiles || gemm_workspace_bytes(p) >= (1ull << 31)))
     return hipErrorInvalidValue;
   if (pr.wf == kWfInt4) return launch_gemm4<kWfInt4>(p.cfg, ka, stream);
   if (pr.wf == kWfInt4Grp) return launch_gemm4<kWfInt4Grp>(p.cfg, ka, stream);

@@ -134,6 +134,48 @@ def test_last_tiles_parity(row):
             assert rep.ok, str(rep)
 
 
+def _unsplit(x, packed, scale, n):
+    """The launch without a workspace: every tile whole."""
+    import ctypes
+    m, k = x.shape
+    y = torch.empty(m, n, dtype=torch.float16, device=x.device)
+    projs = (capi.Proj * 1)(capi.Proj(packed.data_ptr(), scale.data_ptr(), None, y.data_ptr(), n, n))
+    st = capi.load().rf_w8a16_linear_multi(
+        x.data_ptr(), k, 1, projs, 1, m, k, 0, None, 0,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == capi.OK, capi.status_str(st)
+    return y
+
+
+def _big(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    q = torch.randint(-127, 128, (n, k), generator=g, device="cuda", dtype=torch.int8)
+    s = (torch.rand(n, generator=g, device="cuda") * 1e-3 + 1e-4).half()
+    return x, q, s
+
+
+@pytest.mark.gpu
+def test_last_tiles_of_a_launch_beyond_the_counters():
+    """More tiles (16416) than split-K counters (16384), 32 of them past the
+    whole rounds: only those have counters."""
+    m, n, k = 4096, 131328, 3072
+    print(f"last tiles M={m} N={n} K={k}", flush=True)
+    tiles, rem = m // 128 * (n // 256), 32
+    assert tiles * 4 > capi.WS_COUNTER_BYTES and tiles % 256 == rem
+    x, q, s = _big(m, n, k)
+    packed = rf.pack_weight(q)
+    y, whole = rf.linear(x, packed, s), _unsplit(x, packed, s, n)
+    torch.cuda.synchronize()
+    assert int((y != whole).sum()) <= rem * 128 * 256  # elsewhere the same sums
+    rows = np.unique(np.linspace(0, m - 1, 7).astype(int))
+    cols = np.unique(np.r_[np.arange(5, n, 1021), n - 256:n])
+    xc, qc, sc = (t.cpu().numpy() for t in (x[rows], q[cols], s[cols]))
+    rep = o.check_tolerance(y[rows][:, cols].cpu().numpy(), o.cpu_path(xc, qc, sc),
+                            o.oracle_fp64(xc, qc, sc))
+    assert rep.ok, str(rep)
+
+
 @pytest.mark.parametrize("row", INT4_ROWS, ids=_id)
 def test_int4_plan(row):
     m, ns, k, gs, name, splits = row
