@@ -109,13 +109,21 @@ WorkspaceCache& workspace_cache() {
 // launches anything; only then is the size the shape needs queried (a second
 // launch plan), the buffer grown and the call repeated.
 // From M rows on where the GEMM may split the K range of its last tiles only if
-// there is room (it runs them whole otherwise), the size is queried up front.
+// there is room (it runs them whole otherwise), the size is queried up front --
+// except under graph capture, where only a launch that cannot run without it
+// grows the buffer: a buffer allocated there is zeroed by the graph's replays
+// alone, so eager calls before the first replay would find it unset.
 constexpr int64_t kQueryRows = 129;
+bool capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) == hipSuccess &&
+         st != hipStreamCaptureStatusNone;
+}
 template <typename Call, typename Need>
 int with_workspace(const at::Device& dev, void* stream, int64_t M, const char* op, Call call,
                    Need need) {
   WorkspaceCache& wc = workspace_cache();
-  at::Tensor ws = wc.get(dev, stream, M >= kQueryRows ? need() : 0);
+  at::Tensor ws = wc.get(dev, stream, M >= kQueryRows && !capturing(stream) ? need() : 0);
   int st = call(ws.data_ptr(), (size_t)ws.numel());
   if (st == RF_W8A16_EWORKSPACE) {
     const size_t bytes = need();

@@ -176,6 +176,36 @@ def test_last_tiles_of_a_launch_beyond_the_counters():
     assert rep.ok, str(rep)
 
 
+@pytest.mark.gpu
+def test_last_tiles_under_capture():
+    """A capture does not grow the stream's workspace for the split of the last
+    tiles: it runs them whole, and an eager call before the first replay finds
+    cleared counters."""
+    m, n, k = 1300, 24576, 3072
+    print(f"last tiles under capture M={m} N={n} K={k}", flush=True)
+    x, q, s = _big(m, n, k)
+    packed = rf.pack_weight(q)
+    split, whole = rf.linear(x, packed, s), _unsplit(x, packed, s, n)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        rf.linear(x[:1], packed, s)  # the stream's workspace at its least size
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        y = rf.linear(x, packed, s)
+    with torch.cuda.stream(stream):
+        eager = rf.linear(x, packed, s)
+    torch.cuda.synchronize()
+    assert torch.equal(eager, split)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, whole)
+        assert torch.equal(rf.linear(x, packed, s), split)
+
+
 @pytest.mark.parametrize("row", INT4_ROWS, ids=_id)
 def test_int4_plan(row):
     m, ns, k, gs, name, splits = row
