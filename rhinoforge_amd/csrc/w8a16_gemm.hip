@@ -789,7 +789,7 @@ void w8a16_gemm_v3_kernel(GemmKernelArgs a) {
 // True when the 32-bit DMA offsets of w8a16_gemm_v3_kernel cannot overflow
 // for any projection of the launch.
 inline bool v3_offsets_fit(const GemmKernelArgs& ka, int bm, int bn) {
-  const uint64_t a_span = (uint64_t)bm * (uint64_t)ka.ldx * 2 + (uint64_t)round_up(ka.K, kTileK4) * 2;
+  const uint64_t a_span = (uint64_t)bm * (uint64_t)ka.ldx * 2 + (uint64_t)round_up(ka.K, 64) * 2;
   const uint64_t b_span = (uint64_t)(bn / 16) * (uint64_t)ka.wtiles * kTileBytes;
   return a_span < (1ull << 32) && b_span < (1ull << 32);
 }
