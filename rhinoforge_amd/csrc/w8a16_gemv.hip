@@ -479,6 +479,9 @@ __global__ __launch_bounds__(W * 64) void w8a16_gemv_kernel(GemvKernelArgs a) {
   auto load_stage = [&](int st, uint4 (&wv)[U][NS], half8 (&xv)[XR ? U : 1][MT][XN],
                         _Float16 (&sv)[GS ? U : 1][NS], int nvalid) {
     if constexpr (XD) {  // ahead of the stage's weights: their wait then covers the x tiles
+      // The fragment reads of the stage that used this buffer before have
+      // returned once they are waited for: nothing else orders them with the DMA.
+      __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (u >= nvalid) break;  // wave-uniform
