@@ -235,6 +235,32 @@ int rf_w8a16_linear_multi(const void* x, int64_t ldx, int32_t layout, const rf_w
                           int32_t count, int64_t M, int64_t K, int32_t kernel, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* The workspace in two parts, for callers that keep one per stream and let it
+ * grow.  The counters must stay the same memory for as long as calls on the
+ * stream or graphs captured on it may run (zero before the first use, left
+ * zero by every call); the partials need no clearing, so a larger buffer may
+ * replace them at any time, also under graph capture (the old one stays
+ * allocated while a graph refers to it). */
+typedef struct rf_w8a16_scratch {
+  void* counters;       /* RF_W8A16_WS_COUNTER_BYTES bytes, 256-byte aligned */
+  void* partials;       /* 256-byte aligned */
+  size_t partial_bytes; /* rf_w8a16_workspace_bytes*() - RF_W8A16_WS_COUNTER_BYTES suffices */
+} rf_w8a16_scratch;
+
+/* rf_w8a16_linear_multi with such a workspace. */
+int rf_w8a16_linear_multi_scratch(const void* x, int64_t ldx, int32_t layout,
+                                  const rf_w8a16_proj* projs, int32_t count, int64_t M, int64_t K,
+                                  int32_t kernel, const rf_w8a16_scratch* scratch, void* stream);
+
+/* Counters for `stream` on the current device, owned by the library: cleared
+ * since it was loaded, the same memory on every call, never freed.  Nothing is
+ * launched, so a stream that is being captured may ask for them too (counters
+ * cleared by a fill on such a stream would be cleared by the graph's replays
+ * only).  The first RF_W8A16_COUNTER_REGIONS streams of a device that ask get
+ * a region each, later ones RF_W8A16_ESCRATCH. */
+#define RF_W8A16_COUNTER_REGIONS 128
+int rf_w8a16_stream_counters(void* stream, void** counters);
+
 /* No-allocation variant of rf_w8a16_linear_multi.  It has no counterpart in
  * the reference: it is for callers that cannot allocate device memory --
  * code under HIP graph capture, tight serving loops, harnesses that forbid
@@ -280,6 +306,10 @@ int rf_w8a16_linear_argmax(const void* x, int64_t ldx, const void* w_packed, int
                            int32_t* index, int64_t M, int64_t N, int64_t K, void* workspace,
                            size_t workspace_bytes, void* stream);
 size_t rf_w8a16_workspace_bytes_argmax(int64_t M, int64_t N, int64_t K);
+int rf_w8a16_linear_argmax_scratch(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
+                                   const void* scale, const void* bias, void* y, int64_t ldy,
+                                   int32_t* index, int64_t M, int64_t N, int64_t K,
+                                   const rf_w8a16_scratch* scratch, void* stream);
 
 /* ---------------------------------------------------------------------------
  * W4A16: packed int4 weights, per-channel or group-wise fp16 scales, on the
@@ -350,6 +380,9 @@ int rf_w4a16_linear(const void* x, int64_t ldx, const void* w_packed, const void
 int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs, int32_t count,
                           int32_t group_size, int64_t M, int64_t K, int32_t kernel,
                           void* workspace, size_t workspace_bytes, void* stream);
+int rf_w4a16_linear_multi_scratch(const void* x, int64_t ldx, const rf_w8a16_proj* projs,
+                                  int32_t count, int32_t group_size, int64_t M, int64_t K,
+                                  int32_t kernel, const rf_w8a16_scratch* scratch, void* stream);
 
 #ifdef __cplusplus
 } /* extern "C" */

@@ -28,6 +28,7 @@ KERNEL_AUTO = 0
 KERNEL_GEMV = 1
 KERNEL_GEMM = 2
 WS_COUNTER_BYTES = 65536
+COUNTER_REGIONS = 128
 MAX_PROJ = 4
 
 
@@ -49,6 +50,13 @@ class PlanInfo(ctypes.Structure):
                 ("tile_n", ctypes.c_int32), ("splits", ctypes.c_int32),
                 ("waves", ctypes.c_int32), ("workgroups", ctypes.c_int32),
                 ("workspace_bytes", ctypes.c_uint64), ("name", ctypes.c_char * 48)]
+
+
+class Scratch(ctypes.Structure):
+    """struct rf_w8a16_scratch (include/w8a16.h)."""
+    _fields_ = [("counters", ctypes.c_void_p), ("partials", ctypes.c_void_p),
+                ("partial_bytes", ctypes.c_size_t)]
+
 
 # name -> (restype, argtypes): every entry point declared in include/w8a16.h
 _c = ctypes
@@ -74,6 +82,11 @@ SIGNATURES = {
     "rf_w8a16_linear_multi_noalloc": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_int32,
                                                  _c.POINTER(Proj), _c.c_int32, _c.c_int64,
                                                  _c.c_int64, _c.c_int32, _c.c_void_p]),
+    "rf_w8a16_linear_multi_scratch": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_int32,
+                                                 _c.POINTER(Proj), _c.c_int32, _c.c_int64,
+                                                 _c.c_int64, _c.c_int32, _c.POINTER(Scratch),
+                                                 _c.c_void_p]),
+    "rf_w8a16_stream_counters": (_c.c_int, [_c.c_void_p, _c.POINTER(_c.c_void_p)]),
     "rf_w8a16_linear": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int32,
                                    _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int64,
                                    _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int32,
@@ -82,6 +95,10 @@ SIGNATURES = {
                                           _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int64,
                                           _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64,
                                           _c.c_void_p, _c.c_size_t, _c.c_void_p]),
+    "rf_w8a16_linear_argmax_scratch": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int32,
+                                                  _c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_int64,
+                                                  _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64,
+                                                  _c.POINTER(Scratch), _c.c_void_p]),
     "rf_w8a16_workspace_bytes_argmax": (_c.c_size_t, [_c.c_int64, _c.c_int64, _c.c_int64]),
     "rf_w8a16_quantize_device": (_c.c_int, [_c.c_void_p, _c.c_int32, _c.c_int64, _c.c_int64,
                                             _c.c_int64, _c.c_int32, _c.c_int32, _c.c_int32,
@@ -102,6 +119,9 @@ SIGNATURES = {
     "rf_w4a16_linear_multi": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.POINTER(Proj), _c.c_int32,
                                          _c.c_int32, _c.c_int64, _c.c_int64, _c.c_int32,
                                          _c.c_void_p, _c.c_size_t, _c.c_void_p]),
+    "rf_w4a16_linear_multi_scratch": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.POINTER(Proj),
+                                                 _c.c_int32, _c.c_int32, _c.c_int64, _c.c_int64,
+                                                 _c.c_int32, _c.POINTER(Scratch), _c.c_void_p]),
     "rf_w4a16_linear": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p,
                                    _c.c_int32, _c.c_void_p, _c.c_void_p, _c.c_int64,
                                    _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int32,

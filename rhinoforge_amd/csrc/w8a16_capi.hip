@@ -281,7 +281,36 @@ int noalloc_scratch(hipStream_t stream, void** out) {
   return RF_W8A16_OK;
 }
 
+// A caller's scratch: split-K counters and `bytes` of partials.
+struct CallScratch {
+  void* counters = nullptr;
+  void* partials = nullptr;
+  size_t bytes = 0;
+
+  bool holds(size_t need) const {
+    return counters && partials && bytes >= need && aligned(counters, 256) && aligned(partials, 256);
+  }
+  rf::Scratch args() const { return {static_cast<uint32_t*>(counters), static_cast<float*>(partials)}; }
+};
+
+// The one-buffer form: [counters | partials].
+CallScratch of_workspace(void* workspace, size_t bytes) {
+  if (!workspace || bytes < RF_W8A16_WS_COUNTER_BYTES) return {};
+  return {workspace, static_cast<uint8_t*>(workspace) + RF_W8A16_WS_COUNTER_BYTES,
+          bytes - RF_W8A16_WS_COUNTER_BYTES};
+}
+
+CallScratch of_scratch(const rf_w8a16_scratch* s) {
+  if (!s) return {};
+  return {s->counters, s->partials, s->partial_bytes};
+}
+
 }  // namespace
+
+// Counter regions of rf_w8a16_stream_counters: zero when the code object loads
+// (no initializer), so a stream first seen under graph capture needs no fill.
+static __device__ __align__(256)
+    uint8_t counter_regions[RF_W8A16_COUNTER_REGIONS * RF_W8A16_WS_COUNTER_BYTES];
 
 extern "C" {
 
@@ -513,12 +542,11 @@ size_t rf_w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return rf_w8a16_workspace_bytes_multi(M, &N, 1, K);
 }
 
-// rf_w8a16_linear_multi and its no-allocation variant (noalloc: the
-// workspace arguments are ignored and the library's scratch array is used).
+// rf_w8a16_linear_multi and its variants (noalloc: `ws` is ignored and the
+// library's scratch array is used).
 static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
                              const rf_w8a16_proj* projs, int32_t count, int64_t M, int64_t K,
-                             int32_t kernel, void* workspace, size_t workspace_bytes, void* stream,
-                             bool noalloc) {
+                             int32_t kernel, CallScratch ws, void* stream, bool noalloc) {
   if (!x || !projs || count < 1 || count > RF_W8A16_MAX_PROJ) return RF_W8A16_EINVAL;
   if (M < 1 || M > kMaxDim || K < 1 || K > kMaxDim || ldx < K) return RF_W8A16_EINVAL;
   for (int i = 0; i < count; ++i) {
@@ -554,9 +582,10 @@ static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
     return RF_W8A16_EKERNEL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (noalloc) {
-    st = noalloc_scratch(s, &workspace);
+    void* p = nullptr;
+    st = noalloc_scratch(s, &p);
     if (st != RF_W8A16_OK) return st;
-    workspace_bytes = RF_W8A16_NOALLOC_SCRATCH_BYTES;
+    ws = of_workspace(p, RF_W8A16_NOALLOC_SCRATCH_BYTES);
   }
   // A plan needing more workspace than is at hand: the caller's buffer is too
   // small (EWORKSPACE), or the library's fixed scratch is (ESCRATCH).
@@ -579,22 +608,17 @@ static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
     d.N = (int)projs[i].N;
     n32[i] = d.N;
   }
-  auto workspace_ok = [&](size_t extra) {
-    return workspace && workspace_bytes >= RF_W8A16_WS_COUNTER_BYTES + extra &&
-           aligned(workspace, 256);
-  };
   hipError_t e;
   if (kernel == RF_W8A16_KERNEL_GEMV) {
     const rf::GemvPlan p = rf::plan_gemv(pr.M, n32, count, pr.K, dev);
-    if (p.splits > 1 && !workspace_ok(rf::gemv_workspace_bytes(p, pr.M, n32, count)))
-      return too_small;
-    e = rf::launch_gemv(pr, p, p.splits > 1 ? workspace : nullptr, s);
+    if (p.splits > 1 && !ws.holds(rf::gemv_workspace_bytes(p, pr.M, n32, count))) return too_small;
+    e = rf::launch_gemv(pr, p, ws.args(), s);
   } else {
     rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev);
     // (the split of the last tiles is left out where its scratch is missing)
-    if (p.rem_splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
-    if (const size_t extra = rf::gemm_workspace_bytes(p); extra && !workspace_ok(extra)) return too_small;
-    e = rf::launch_gemm(pr, p, rf::gemm_workspace_bytes(p) ? workspace : nullptr, s);
+    if (p.rem_splits > 1 && !ws.holds(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
+    if (const size_t need = rf::gemm_workspace_bytes(p); need && !ws.holds(need)) return too_small;
+    e = rf::launch_gemm(pr, p, ws.args(), s);
   }
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
 }
@@ -602,14 +626,45 @@ static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
 int rf_w8a16_linear_multi(const void* x, int64_t ldx, int32_t layout, const rf_w8a16_proj* projs,
                           int32_t count, int64_t M, int64_t K, int32_t kernel, void* workspace,
                           size_t workspace_bytes, void* stream) {
-  return linear_multi_impl(x, ldx, layout, projs, count, M, K, kernel, workspace, workspace_bytes,
-                           stream, false);
+  return linear_multi_impl(x, ldx, layout, projs, count, M, K, kernel,
+                           of_workspace(workspace, workspace_bytes), stream, false);
+}
+
+int rf_w8a16_linear_multi_scratch(const void* x, int64_t ldx, int32_t layout,
+                                  const rf_w8a16_proj* projs, int32_t count, int64_t M, int64_t K,
+                                  int32_t kernel, const rf_w8a16_scratch* scratch, void* stream) {
+  return linear_multi_impl(x, ldx, layout, projs, count, M, K, kernel, of_scratch(scratch), stream,
+                           false);
+}
+
+// Regions are taken in order and kept: a stream's counters are zero between its
+// calls, so a handle that HIP hands out again may share them.
+int rf_w8a16_stream_counters(void* stream, void** counters) {
+  constexpr int kMaxDevices = 64;
+  static std::mutex mu;
+  static void* owner[kMaxDevices][RF_W8A16_COUNTER_REGIONS];
+  static int used[kMaxDevices];
+  if (!counters) return RF_W8A16_EINVAL;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return RF_W8A16_EHIP;
+  if (dev < 0 || dev >= kMaxDevices) return RF_W8A16_EDEVICE;
+  std::lock_guard<std::mutex> g(mu);
+  int r = 0;
+  while (r < used[dev] && owner[dev][r] != stream) ++r;
+  if (r == RF_W8A16_COUNTER_REGIONS) return RF_W8A16_ESCRATCH;
+  void* base = nullptr;
+  if (hipGetSymbolAddress(&base, HIP_SYMBOL(counter_regions)) != hipSuccess || !base ||
+      !aligned(base, 256))
+    return RF_W8A16_EHIP;
+  if (r == used[dev]) owner[dev][used[dev]++] = stream;
+  *counters = static_cast<uint8_t*>(base) + (size_t)r * RF_W8A16_WS_COUNTER_BYTES;
+  return RF_W8A16_OK;
 }
 
 int rf_w8a16_linear_multi_noalloc(const void* x, int64_t ldx, int32_t layout,
                                   const rf_w8a16_proj* projs, int32_t count, int64_t M, int64_t K,
                                   int32_t kernel, void* stream) {
-  return linear_multi_impl(x, ldx, layout, projs, count, M, K, kernel, nullptr, 0, stream, true);
+  return linear_multi_impl(x, ldx, layout, projs, count, M, K, kernel, {}, stream, true);
 }
 
 int rf_w8a16_linear(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
@@ -717,9 +772,9 @@ size_t rf_w4a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return rf_w4a16_workspace_bytes_multi(M, &N, 1, K);
 }
 
-int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs, int32_t count,
-                          int32_t group_size, int64_t M, int64_t K, int32_t kernel,
-                          void* workspace, size_t workspace_bytes, void* stream) {
+static int w4_linear_multi_impl(const void* x, int64_t ldx, const rf_w8a16_proj* projs,
+                                int32_t count, int32_t group_size, int64_t M, int64_t K,
+                                int32_t kernel, CallScratch ws, void* stream) {
   if (!x || !projs || count < 1 || count > RF_W8A16_MAX_PROJ) return RF_W8A16_EINVAL;
   if (M < 1 || M > kMaxDim || K < 1 || K > kMaxDim || ldx < K) return RF_W8A16_EINVAL;
   if (group_size != 0 && group_size != 32 && group_size != 64 && group_size != 128)
@@ -769,25 +824,36 @@ int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs
     d.ldy = projs[i].ldy;
     d.N = (int)projs[i].N;
   }
-  auto workspace_ok = [&](size_t extra) {
-    return workspace && workspace_bytes >= RF_W8A16_WS_COUNTER_BYTES + extra &&
-           aligned(workspace, 256);
-  };
   hipError_t e;
   if (kernel == RF_W8A16_KERNEL_GEMV) {
     const rf::GemvPlan p = rf::plan_gemv_int4(pr.M, n32, count, pr.K, group_size != 0, dev);
-    if (p.splits > 1 && !workspace_ok(rf::gemv_workspace_bytes(p, pr.M, n32, count)))
+    if (p.splits > 1 && !ws.holds(rf::gemv_workspace_bytes(p, pr.M, n32, count)))
       return RF_W8A16_EWORKSPACE;
-    e = rf::launch_gemv(pr, p, p.splits > 1 ? workspace : nullptr, s);
+    e = rf::launch_gemv(pr, p, ws.args(), s);
   } else {
     rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev, true);
-    if (p.rem_splits > 1 && !workspace_ok(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
+    if (p.rem_splits > 1 && !ws.holds(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
     // The int4 GEMM has no 64-bit-address kernel.
     if (!rf::gemm_offsets_fit(p, ldx, pr.K, true)) return RF_W8A16_EKERNEL;
-    if (const size_t extra = rf::gemm_workspace_bytes(p); extra && !workspace_ok(extra)) return RF_W8A16_EWORKSPACE;
-    e = rf::launch_gemm(pr, p, rf::gemm_workspace_bytes(p) ? workspace : nullptr, s);
+    if (const size_t need = rf::gemm_workspace_bytes(p); need && !ws.holds(need))
+      return RF_W8A16_EWORKSPACE;
+    e = rf::launch_gemm(pr, p, ws.args(), s);
   }
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
+}
+
+int rf_w4a16_linear_multi(const void* x, int64_t ldx, const rf_w8a16_proj* projs, int32_t count,
+                          int32_t group_size, int64_t M, int64_t K, int32_t kernel,
+                          void* workspace, size_t workspace_bytes, void* stream) {
+  return w4_linear_multi_impl(x, ldx, projs, count, group_size, M, K, kernel,
+                              of_workspace(workspace, workspace_bytes), stream);
+}
+
+int rf_w4a16_linear_multi_scratch(const void* x, int64_t ldx, const rf_w8a16_proj* projs,
+                                  int32_t count, int32_t group_size, int64_t M, int64_t K,
+                                  int32_t kernel, const rf_w8a16_scratch* scratch, void* stream) {
+  return w4_linear_multi_impl(x, ldx, projs, count, group_size, M, K, kernel, of_scratch(scratch),
+                              stream);
 }
 
 int rf_w4a16_linear(const void* x, int64_t ldx, const void* w_packed, const void* scale,
@@ -819,10 +885,10 @@ size_t rf_w8a16_workspace_bytes_argmax(int64_t M, int64_t N, int64_t K) {
          rf::argmax_slot_bytes(p, (int)M);
 }
 
-int rf_w8a16_linear_argmax(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
-                           const void* scale, const void* bias, void* y, int64_t ldy,
-                           int32_t* index, int64_t M, int64_t N, int64_t K, void* workspace,
-                           size_t workspace_bytes, void* stream) {
+static int linear_argmax_impl(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
+                              const void* scale, const void* bias, void* y, int64_t ldy,
+                              int32_t* index, int64_t M, int64_t N, int64_t K,
+                              const CallScratch& ws, void* stream) {
   if (!x || !w_packed || !scale || !index) return RF_W8A16_EINVAL;
   if (M < 1 || M > kMaxDim || check_nk(N, K) != RF_W8A16_OK || ldx < K) return RF_W8A16_EINVAL;
   if (N > INT32_MAX - 1 || (y && ldy < N)) return RF_W8A16_EINVAL;
@@ -851,15 +917,30 @@ int rf_w8a16_linear_argmax(const void* x, int64_t ldx, const void* w_packed, int
   pr.proj[0].N = (int)N;
   const int n32 = (int)N;
   const rf::GemvPlan p = rf::plan_gemv(pr.M, &n32, 1, pr.K, dev);
-  const size_t slots_off = RF_W8A16_WS_COUNTER_BYTES +
+  const size_t slots_off =
       (size_t)rf::round_up((int64_t)rf::gemv_workspace_bytes(p, pr.M, &n32, 1), 256);
-  const size_t need = slots_off + rf::argmax_slot_bytes(p, pr.M);
-  if (!workspace || workspace_bytes < need || !aligned(workspace, 256)) return RF_W8A16_EWORKSPACE;
-  rf::ArgmaxTarget am;  // per-workgroup keys in the scratch part of the workspace
-  am.slots = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(workspace) + slots_off);
+  if (!ws.holds(slots_off + rf::argmax_slot_bytes(p, pr.M))) return RF_W8A16_EWORKSPACE;
+  rf::ArgmaxTarget am;  // per-workgroup keys behind the partials
+  am.slots = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(ws.partials) + slots_off);
   am.index = index;
-  const hipError_t e = rf::launch_gemv(pr, p, workspace, static_cast<hipStream_t>(stream), &am);
+  const hipError_t e = rf::launch_gemv(pr, p, ws.args(), static_cast<hipStream_t>(stream), &am);
   return e == hipSuccess ? RF_W8A16_OK : RF_W8A16_EHIP;
+}
+
+int rf_w8a16_linear_argmax(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
+                           const void* scale, const void* bias, void* y, int64_t ldy,
+                           int32_t* index, int64_t M, int64_t N, int64_t K, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  return linear_argmax_impl(x, ldx, w_packed, layout, scale, bias, y, ldy, index, M, N, K,
+                            of_workspace(workspace, workspace_bytes), stream);
+}
+
+int rf_w8a16_linear_argmax_scratch(const void* x, int64_t ldx, const void* w_packed, int32_t layout,
+                                   const void* scale, const void* bias, void* y, int64_t ldy,
+                                   int32_t* index, int64_t M, int64_t N, int64_t K,
+                                   const rf_w8a16_scratch* scratch, void* stream) {
+  return linear_argmax_impl(x, ldx, w_packed, layout, scale, bias, y, ldy, index, M, N, K,
+                            of_scratch(scratch), stream);
 }
 
 }  // extern "C"

@@ -1546,7 +1546,7 @@ size_t gemm_workspace_bytes(const GemmPlan& p) {
   return parts * (size_t)p.bm * (size_t)p.bn * sizeof(float);
 }
 
-hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* workspace,
+hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, const Scratch& scratch,
                        hipStream_t stream) {
   GemmPlan p = plan;
   if (pr.nproj < 1 || pr.nproj > kMaxProj) return hipErrorInvalidValue;
@@ -1590,12 +1590,8 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
     ka.rem0 = q.rem0;
     ka.rem_splits = q.rem_splits;
     ka.rem_kb = q.rem_kb;
-    ka.partial = nullptr;
-    ka.counters = nullptr;
-    if (q.splits > 1 || q.rem_splits > 1) {
-      ka.counters = static_cast<uint32_t*>(workspace);
-      ka.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + RF_W8A16_WS_COUNTER_BYTES);
-    }
+    ka.partial = scratch.partial;
+    ka.counters = scratch.counters;
   };
   // 64-bit addressing where the v3 kernels' 32-bit tile offsets could
   // overflow (int8; int4 has no such kernel and its callers refuse first).
@@ -1607,7 +1603,8 @@ hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& plan, void* work
   // (of a launch that splits its last tiles only those have counters)
   const int64_t split_tiles = (int64_t)p.tiles_m * p.tiles_n - (p.rem_splits > 1 ? p.rem0 : 0);
   if ((p.splits > 1 || p.rem_splits > 1) &&
-      (!workspace || split_tiles > kMaxSplitTiles || gemm_workspace_bytes(p) >= (1ull << 31)))
+      (!scratch.counters || !scratch.partial || split_tiles > kMaxSplitTiles ||
+       gemm_workspace_bytes(p) >= (1ull << 31)))
     return hipErrorInvalidValue;
   if (pr.wf == kWfInt4) return launch_gemm4<kWfInt4>(p.cfg, ka, stream);
   if (pr.wf == kWfInt4Grp) return launch_gemm4<kWfInt4Grp>(p.cfg, ka, stream);

@@ -838,7 +838,7 @@ hipError_t launch_1(const GemvKernelArgs& ka, const GemvPlan& p, hipStream_t str
   return launch_t<1, 1, W, U, false, true, WF>(ka, p, stream);
 }
 
-GemvKernelArgs make_args(const LinearProblem& pr, const GemvPlan& p, void* workspace) {
+GemvKernelArgs make_args(const LinearProblem& pr, const GemvPlan& p, const Scratch& scratch) {
   GemvKernelArgs ka;
   ka.x = pr.x;
   ka.ldx = pr.ldx;
@@ -871,11 +871,8 @@ GemvKernelArgs make_args(const LinearProblem& pr, const GemvPlan& p, void* works
   ka.splits = p.splits;
   ka.kb_per_split = p.kb_per_split;
   ka.np = col;
-  // Workspace: [counters | partials]; counter region size fixed by the ABI.
-  ka.counters = reinterpret_cast<uint32_t*>(workspace);
-  ka.partial = workspace ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) +
-                                                    RF_W8A16_WS_COUNTER_BYTES)
-                         : nullptr;
+  ka.counters = scratch.counters;
+  ka.partial = scratch.partial;
   ka.amax_slots = nullptr;
   // Contiguous strip ranges per XCD on every group-wise launch: without them
   // each XCD's L2 fetches the scale lines of its strips' neighbours too
@@ -1022,10 +1019,10 @@ size_t gemv_workspace_bytes(const GemvPlan& p, int M, const int* Ns, int nproj) 
   return (size_t)p.splits * (size_t)M * (size_t)np * sizeof(float);
 }
 
-hipError_t launch_gemv(const LinearProblem& pr, const GemvPlan& p, void* workspace,
+hipError_t launch_gemv(const LinearProblem& pr, const GemvPlan& p, const Scratch& scratch,
                        hipStream_t stream, const ArgmaxTarget* am) {
   if (pr.nproj < 1 || pr.nproj > kMaxProj) return hipErrorInvalidValue;
-  GemvKernelArgs ka = make_args(pr, p, workspace);
+  GemvKernelArgs ka = make_args(pr, p, scratch);
   if (pr.wf != kWfInt8) {
     if (am) return hipErrorInvalidValue;
     return pr.wf == kWfInt4 ? launch_gemv4_cfg<kWfInt4>(ka, p, stream)

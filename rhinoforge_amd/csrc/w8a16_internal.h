@@ -116,10 +116,17 @@ size_t argmax_slot_bytes(const GemvPlan& p, int M);
 // zero-between-calls counter region at the start of every workspace.
 constexpr int kMaxSplitCounters = (int)(RF_W8A16_WS_COUNTER_BYTES / 4);
 
+// What a K-split launch uses: the counters, zero between calls, and fp32
+// partials of gemv_ / gemm_workspace_bytes (both null where nothing is split).
+struct Scratch {
+  uint32_t* counters = nullptr;
+  float* partial = nullptr;
+};
+
 // Launchers: return hipSuccess or the launch error.
-hipError_t launch_gemv(const LinearProblem& pr, const GemvPlan& p, void* workspace,
+hipError_t launch_gemv(const LinearProblem& pr, const GemvPlan& p, const Scratch& scratch,
                        hipStream_t stream, const ArgmaxTarget* am = nullptr);
-hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& p, void* workspace,
+hipError_t launch_gemm(const LinearProblem& pr, const GemmPlan& p, const Scratch& scratch,
                        hipStream_t stream);
 hipError_t launch_pack4(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* dst,
                         hipStream_t stream);

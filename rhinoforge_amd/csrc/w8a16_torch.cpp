@@ -73,63 +73,89 @@ void check_packed(const at::Tensor& packed, at::ScalarType dtype,
               ", got ", packed.sizes());
 }
 
-// Workspace per (device, stream): allocated through torch's caching
-// allocator, zero-filled once (fill kernel), at least kMinWorkspace bytes.
-// The C ABI leaves its counter region zero after every call, and calls on
-// one stream are ordered, so one buffer per stream is safe to reuse.  A
-// buffer that has to grow is retired, never freed: a HIP graph captured
-// earlier on that stream may still reference it.
-constexpr int64_t kMinWorkspace = 16 << 20;
+// Scratch per (device, stream), in two parts (the C ABI's rf_w8a16_scratch).
+// Calls on one stream are ordered and leave the counters zero, so one set per
+// stream is safe to reuse.
+//   counters  allocated and cleared once, on the stream itself; for a stream
+//             first seen under graph capture the library's own, which nothing
+//             has to clear.  Never replaced: a fill recorded into a graph would
+//             clear them on that graph's replays only, and every other call on
+//             the stream might find anything.
+//   partials  at least kMinPartials bytes, never cleared.  A buffer that has to
+//             grow, under capture too, is retired, never freed: a HIP graph
+//             captured earlier on that stream may still reference it.
+constexpr int64_t kMinPartials = 16 << 20;
 
-struct WorkspaceCache {
-  std::mutex mu;
-  std::map<std::pair<int, void*>, at::Tensor> bufs;
-  std::vector<at::Tensor> retired;
-
-  at::Tensor get(const at::Device& dev, void* stream, size_t bytes) {
-    std::lock_guard<std::mutex> g(mu);
-    auto key = std::make_pair((int)dev.index(), stream);
-    auto it = bufs.find(key);
-    if (it != bufs.end() && (size_t)it->second.numel() >= bytes) return it->second;
-    if (it != bufs.end()) retired.push_back(it->second);
-    const int64_t sz = ceil_to(std::max<int64_t>((int64_t)bytes, kMinWorkspace), 1 << 20);
-    at::Tensor t = at::zeros({sz}, at::TensorOptions().dtype(at::kByte).device(dev));
-    bufs[key] = t;
-    return t;
-  }
-};
-
-WorkspaceCache& workspace_cache() {
-  static WorkspaceCache* c = new WorkspaceCache();  // lives until process exit
-  return *c;
-}
-
-// Runs call(workspace, bytes) with the stream's cached workspace.  The C ABI
-// refuses a workspace that is too small with RF_W8A16_EWORKSPACE before it
-// launches anything; only then is the size the shape needs queried (a second
-// launch plan), the buffer grown and the call repeated.
-// From M rows on where the GEMM may split the K range of its last tiles only if
-// there is room (it runs them whole otherwise), the size is queried up front --
-// except under graph capture, where only a launch that cannot run without it
-// grows the buffer: a buffer allocated there is zeroed by the graph's replays
-// alone, so eager calls before the first replay would find it unset.
-constexpr int64_t kQueryRows = 129;
 bool capturing(void* stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) == hipSuccess &&
          st != hipStreamCaptureStatusNone;
 }
+
+struct ScratchCache {
+  std::mutex mu;
+  std::map<std::pair<int, void*>, rf_w8a16_scratch> sets;
+  std::vector<at::Tensor> kept;  // every buffer handed out, until the process ends
+
+  void* keep(at::Tensor t) {
+    kept.push_back(t);
+    return t.data_ptr();
+  }
+
+  // The stream's scratch with at least `bytes` of partials (current device: dev).
+  rf_w8a16_scratch get(const at::Device& dev, void* stream, size_t bytes, const char* op) {
+    std::lock_guard<std::mutex> g(mu);
+    rf_w8a16_scratch& s = sets[std::make_pair((int)dev.index(), stream)];
+    const auto opts = at::TensorOptions().dtype(at::kByte).device(dev);
+    if (!s.counters) {
+      if (capturing(stream)) {
+        const int st = rf_w8a16_stream_counters(stream, &s.counters);
+        TORCH_CHECK(st == RF_W8A16_OK, op, ": no split-K counters for a stream first used under "
+                    "graph capture (status ", st, "); make one call on it before the capture "
+                    "begins");
+      } else {
+        s.counters = keep(at::zeros({RF_W8A16_WS_COUNTER_BYTES}, opts));
+      }
+    }
+    if (!s.partials || s.partial_bytes < bytes) {
+      const int64_t sz = ceil_to(std::max<int64_t>((int64_t)bytes, kMinPartials), 1 << 20);
+      s.partials = keep(at::empty({sz}, opts));
+      s.partial_bytes = (size_t)sz;
+    }
+    return s;
+  }
+};
+
+ScratchCache& scratch_cache() {
+  static ScratchCache* c = new ScratchCache();  // lives until process exit
+  return *c;
+}
+
+// Runs call(scratch) with the stream's cached scratch.  The C ABI refuses one
+// that is too small with RF_W8A16_EWORKSPACE before it launches anything; only
+// then is the size the shape needs queried (a second launch plan: need()
+// returns the one-buffer size, counters included), the partials grown and the
+// call repeated.
+// From M rows on where the GEMM may split the K range of its last tiles only if
+// there is room (it runs them whole otherwise), the size is queried up front,
+// except under graph capture.
+constexpr int64_t kQueryRows = 129;
 template <typename Call, typename Need>
-int with_workspace(const at::Device& dev, void* stream, int64_t M, const char* op, Call call,
-                   Need need) {
-  WorkspaceCache& wc = workspace_cache();
-  at::Tensor ws = wc.get(dev, stream, M >= kQueryRows && !capturing(stream) ? need() : 0);
-  int st = call(ws.data_ptr(), (size_t)ws.numel());
-  if (st == RF_W8A16_EWORKSPACE) {
+int with_scratch(const at::Device& dev, void* stream, int64_t M, const char* op, Call call,
+                 Need need) {
+  ScratchCache& cache = scratch_cache();
+  auto partial_bytes = [&] {
     const size_t bytes = need();
+    return bytes > RF_W8A16_WS_COUNTER_BYTES ? bytes - RF_W8A16_WS_COUNTER_BYTES : 0;
+  };
+  rf_w8a16_scratch s =
+      cache.get(dev, stream, M >= kQueryRows && !capturing(stream) ? partial_bytes() : 0, op);
+  int st = call(&s);
+  if (st == RF_W8A16_EWORKSPACE) {
+    const size_t bytes = partial_bytes();
     TORCH_CHECK(bytes > 0, op, ": ", rf_w8a16_status_str(RF_W8A16_EINVAL));
-    ws = wc.get(dev, stream, bytes);
-    st = call(ws.data_ptr(), (size_t)ws.numel());
+    s = cache.get(dev, stream, bytes, op);
+    st = call(&s);
   }
   return st;
 }
@@ -237,12 +263,12 @@ void launch(const Checked& c, const at::Tensor& weight, const at::Tensor& scale,
   c10::DeviceGuard guard(c.x2.device());
   void* stream = c10::hip::getCurrentHIPStream(c.x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
-  const int st = with_workspace(
+  const rf_w8a16_proj proj{weight.data_ptr(), scale.data_ptr(), bptr, y.data_ptr(), c.N, c.N};
+  const int st = with_scratch(
       c.x2.device(), stream, c.M, op,
-      [&](void* ws, size_t ws_bytes) {
-        return rf_w8a16_linear(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(), (int32_t)layout,
-                               scale.data_ptr(), bptr, y.data_ptr(), c.N, c.M, c.N, c.K,
-                               (int32_t)kernel, ws, ws_bytes, stream);
+      [&](const rf_w8a16_scratch* scratch) {
+        return rf_w8a16_linear_multi_scratch(c.x2.data_ptr(), c.x2.stride(0), (int32_t)layout,
+                                             &proj, 1, c.M, c.K, (int32_t)kernel, scratch, stream);
       },
       [&] { return rf_w8a16_workspace_bytes(c.M, c.N, c.K); });
   check_status(st, op);
@@ -315,12 +341,12 @@ std::vector<at::Tensor> linear_multi_hip(const at::Tensor& input, at::TensorList
   if (c0.M > 0) {
     c10::DeviceGuard guard(c0.x2.device());
     void* stream = c10::hip::getCurrentHIPStream(c0.x2.device().index()).stream();
-    const int st = with_workspace(
+    const int st = with_scratch(
         c0.x2.device(), stream, c0.M, op,
-        [&](void* ws, size_t ws_bytes) {
-          return rf_w8a16_linear_multi(c0.x2.data_ptr(), c0.x2.stride(0), (int32_t)layout, projs,
-                                       (int32_t)count, c0.M, c0.K, (int32_t)kernel, ws, ws_bytes,
-                                       stream);
+        [&](const rf_w8a16_scratch* scratch) {
+          return rf_w8a16_linear_multi_scratch(c0.x2.data_ptr(), c0.x2.stride(0), (int32_t)layout,
+                                               projs, (int32_t)count, c0.M, c0.K, (int32_t)kernel,
+                                               scratch, stream);
         },
         [&] { return rf_w8a16_workspace_bytes_multi(c0.M, Ns, (int32_t)count, c0.K); });
     check_status(st, op);
@@ -470,14 +496,14 @@ std::tuple<at::Tensor, at::Tensor> linear_argmax_hip(const at::Tensor& input,
   c10::DeviceGuard dev_guard(c.x2.device());
   void* stream = c10::hip::getCurrentHIPStream(c.x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
-  const int st = with_workspace(
+  const int st = with_scratch(
       c.x2.device(), stream, c.M, op,
-      [&](void* ws, size_t ws_bytes) {
-        return rf_w8a16_linear_argmax(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(),
-                                      (int32_t)layout, scale.data_ptr(), bptr,
-                                      return_logits ? logits.data_ptr() : nullptr, c.N,
-                                      index.data_ptr<int32_t>(), c.M, c.N, c.K, ws, ws_bytes,
-                                      stream);
+      [&](const rf_w8a16_scratch* scratch) {
+        return rf_w8a16_linear_argmax_scratch(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(),
+                                              (int32_t)layout, scale.data_ptr(), bptr,
+                                              return_logits ? logits.data_ptr() : nullptr, c.N,
+                                              index.data_ptr<int32_t>(), c.M, c.N, c.K, scratch,
+                                              stream);
       },
       [&] { return rf_w8a16_workspace_bytes_argmax(c.M, c.N, c.K); });
   check_status(st, op);
@@ -681,12 +707,13 @@ at::Tensor w4_linear_hip(const at::Tensor& input, const at::Tensor& weight, cons
   c10::DeviceGuard dev_guard(x2.device());
   void* stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
-  const int st = with_workspace(
+  const rf_w8a16_proj proj{weight.data_ptr(), sc.data_ptr(), bptr, y.data_ptr(), N, N};
+  const int st = with_scratch(
       x2.device(), stream, M, op,
-      [&](void* ws, size_t ws_bytes) {
-        return rf_w4a16_linear(x2.data_ptr(), x2.stride(0), weight.data_ptr(), sc.data_ptr(),
-                               (int32_t)group_size, bptr, y.data_ptr(), N, M, N, K,
-                               (int32_t)kernel, ws, ws_bytes, stream);
+      [&](const rf_w8a16_scratch* scratch) {
+        return rf_w4a16_linear_multi_scratch(x2.data_ptr(), x2.stride(0), &proj, 1,
+                                             (int32_t)group_size, M, K, (int32_t)kernel, scratch,
+                                             stream);
       },
       [&] { return rf_w4a16_workspace_bytes(M, N, K); });
   check_status(st, op);
@@ -768,12 +795,12 @@ std::vector<at::Tensor> w4_linear_multi_hip(const at::Tensor& input, at::TensorL
   const at::Tensor x2 = compact_rows(input.dim() == 2 ? input : input.reshape({M, K}));
   c10::DeviceGuard dev_guard(x2.device());
   void* stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
-  const int st = with_workspace(
+  const int st = with_scratch(
       x2.device(), stream, M, op,
-      [&](void* ws, size_t ws_bytes) {
-        return rf_w4a16_linear_multi(x2.data_ptr(), x2.stride(0), projs, (int32_t)count,
-                                     (int32_t)group_size, M, K, (int32_t)kernel, ws, ws_bytes,
-                                     stream);
+      [&](const rf_w8a16_scratch* scratch) {
+        return rf_w4a16_linear_multi_scratch(x2.data_ptr(), x2.stride(0), projs, (int32_t)count,
+                                             (int32_t)group_size, M, K, (int32_t)kernel, scratch,
+                                             stream);
       },
       [&] { return rf_w4a16_workspace_bytes_multi(M, Ns, (int32_t)count, K); });
   check_status(st, op);
