@@ -152,7 +152,8 @@ typedef struct rf_w8a16_plan_info {
   int32_t tile_n;           /* output channels per workgroup, per projection */
   int32_t splits;           /* K splits across workgroups (1: no workspace use); of the
                                last tiles only where workgroups < tiles * splits: those
-                               run unsplit if the workspace lacks workspace_bytes */
+                               run unsplit if the one-buffer workspace lacks
+                               workspace_bytes */
   int32_t waves;            /* wavefronts per workgroup */
   int32_t workgroups;       /* workgroups of the launch, all splits */
   uint64_t workspace_bytes; /* workspace the launch uses past the counter region */
@@ -247,7 +248,10 @@ typedef struct rf_w8a16_scratch {
   size_t partial_bytes; /* rf_w8a16_workspace_bytes*() - RF_W8A16_WS_COUNTER_BYTES suffices */
 } rf_w8a16_scratch;
 
-/* rf_w8a16_linear_multi with such a workspace. */
+/* rf_w8a16_linear_multi with such a workspace.  A launch whose plan needs more
+ * partials returns RF_W8A16_EWORKSPACE and runs nothing, also where
+ * rf_w8a16_linear_multi would leave out the split of its last tiles: the sums,
+ * and so the last bits, of a result do not depend on the size of the buffer. */
 int rf_w8a16_linear_multi_scratch(const void* x, int64_t ldx, int32_t layout,
                                   const rf_w8a16_proj* projs, int32_t count, int64_t M, int64_t K,
                                   int32_t kernel, const rf_w8a16_scratch* scratch, void* stream);

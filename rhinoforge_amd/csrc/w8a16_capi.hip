@@ -281,11 +281,15 @@ int noalloc_scratch(hipStream_t stream, void** out) {
   return RF_W8A16_OK;
 }
 
-// A caller's scratch: split-K counters and `bytes` of partials.
+// A caller's scratch: split-K counters and `bytes` of partials.  required: a
+// launch is refused where its plan needs more (the caller grows the buffer and
+// calls again); otherwise the split of the last tiles, which a launch can run
+// without, is left out there.
 struct CallScratch {
   void* counters = nullptr;
   void* partials = nullptr;
   size_t bytes = 0;
+  bool required = false;
 
   bool holds(size_t need) const {
     return counters && partials && bytes >= need && aligned(counters, 256) && aligned(partials, 256);
@@ -297,12 +301,12 @@ struct CallScratch {
 CallScratch of_workspace(void* workspace, size_t bytes) {
   if (!workspace || bytes < RF_W8A16_WS_COUNTER_BYTES) return {};
   return {workspace, static_cast<uint8_t*>(workspace) + RF_W8A16_WS_COUNTER_BYTES,
-          bytes - RF_W8A16_WS_COUNTER_BYTES};
+          bytes - RF_W8A16_WS_COUNTER_BYTES, false};
 }
 
 CallScratch of_scratch(const rf_w8a16_scratch* s) {
-  if (!s) return {};
-  return {s->counters, s->partials, s->partial_bytes};
+  if (!s) return {nullptr, nullptr, 0, true};
+  return {s->counters, s->partials, s->partial_bytes, true};
 }
 
 }  // namespace
@@ -615,8 +619,8 @@ static int linear_multi_impl(const void* x, int64_t ldx, int32_t layout,
     e = rf::launch_gemv(pr, p, ws.args(), s);
   } else {
     rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev);
-    // (the split of the last tiles is left out where its scratch is missing)
-    if (p.rem_splits > 1 && !ws.holds(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
+    if (p.rem_splits > 1 && !ws.required && !ws.holds(rf::gemm_workspace_bytes(p)))
+      p.rem_splits = 1;
     if (const size_t need = rf::gemm_workspace_bytes(p); need && !ws.holds(need)) return too_small;
     e = rf::launch_gemm(pr, p, ws.args(), s);
   }
@@ -832,7 +836,8 @@ static int w4_linear_multi_impl(const void* x, int64_t ldx, const rf_w8a16_proj*
     e = rf::launch_gemv(pr, p, ws.args(), s);
   } else {
     rf::GemmPlan p = rf::plan_gemm(pr.M, n32, count, pr.K, dev, true);
-    if (p.rem_splits > 1 && !ws.holds(rf::gemm_workspace_bytes(p))) p.rem_splits = 1;
+    if (p.rem_splits > 1 && !ws.required && !ws.holds(rf::gemm_workspace_bytes(p)))
+      p.rem_splits = 1;
     // The int4 GEMM has no 64-bit-address kernel.
     if (!rf::gemm_offsets_fit(p, ldx, pr.K, true)) return RF_W8A16_EKERNEL;
     if (const size_t need = rf::gemm_workspace_bytes(p); need && !ws.holds(need))

@@ -136,25 +136,15 @@ ScratchCache& scratch_cache() {
 // then is the size the shape needs queried (a second launch plan: need()
 // returns the one-buffer size, counters included), the partials grown and the
 // call repeated.
-// From M rows on where the GEMM may split the K range of its last tiles only if
-// there is room (it runs them whole otherwise), the size is queried up front,
-// except under graph capture.
-constexpr int64_t kQueryRows = 129;
 template <typename Call, typename Need>
-int with_scratch(const at::Device& dev, void* stream, int64_t M, const char* op, Call call,
-                 Need need) {
+int with_scratch(const at::Device& dev, void* stream, const char* op, Call call, Need need) {
   ScratchCache& cache = scratch_cache();
-  auto partial_bytes = [&] {
-    const size_t bytes = need();
-    return bytes > RF_W8A16_WS_COUNTER_BYTES ? bytes - RF_W8A16_WS_COUNTER_BYTES : 0;
-  };
-  rf_w8a16_scratch s =
-      cache.get(dev, stream, M >= kQueryRows && !capturing(stream) ? partial_bytes() : 0, op);
+  rf_w8a16_scratch s = cache.get(dev, stream, 0, op);
   int st = call(&s);
   if (st == RF_W8A16_EWORKSPACE) {
-    const size_t bytes = partial_bytes();
-    TORCH_CHECK(bytes > 0, op, ": ", rf_w8a16_status_str(RF_W8A16_EINVAL));
-    s = cache.get(dev, stream, bytes, op);
+    const size_t bytes = need();
+    TORCH_CHECK(bytes > RF_W8A16_WS_COUNTER_BYTES, op, ": ", rf_w8a16_status_str(RF_W8A16_EINVAL));
+    s = cache.get(dev, stream, bytes - RF_W8A16_WS_COUNTER_BYTES, op);
     st = call(&s);
   }
   return st;
@@ -265,7 +255,7 @@ void launch(const Checked& c, const at::Tensor& weight, const at::Tensor& scale,
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const rf_w8a16_proj proj{weight.data_ptr(), scale.data_ptr(), bptr, y.data_ptr(), c.N, c.N};
   const int st = with_scratch(
-      c.x2.device(), stream, c.M, op,
+      c.x2.device(), stream, op,
       [&](const rf_w8a16_scratch* scratch) {
         return rf_w8a16_linear_multi_scratch(c.x2.data_ptr(), c.x2.stride(0), (int32_t)layout,
                                              &proj, 1, c.M, c.K, (int32_t)kernel, scratch, stream);
@@ -342,7 +332,7 @@ std::vector<at::Tensor> linear_multi_hip(const at::Tensor& input, at::TensorList
     c10::DeviceGuard guard(c0.x2.device());
     void* stream = c10::hip::getCurrentHIPStream(c0.x2.device().index()).stream();
     const int st = with_scratch(
-        c0.x2.device(), stream, c0.M, op,
+        c0.x2.device(), stream, op,
         [&](const rf_w8a16_scratch* scratch) {
           return rf_w8a16_linear_multi_scratch(c0.x2.data_ptr(), c0.x2.stride(0), (int32_t)layout,
                                                projs, (int32_t)count, c0.M, c0.K, (int32_t)kernel,
@@ -497,7 +487,7 @@ std::tuple<at::Tensor, at::Tensor> linear_argmax_hip(const at::Tensor& input,
   void* stream = c10::hip::getCurrentHIPStream(c.x2.device().index()).stream();
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const int st = with_scratch(
-      c.x2.device(), stream, c.M, op,
+      c.x2.device(), stream, op,
       [&](const rf_w8a16_scratch* scratch) {
         return rf_w8a16_linear_argmax_scratch(c.x2.data_ptr(), c.x2.stride(0), weight.data_ptr(),
                                               (int32_t)layout, scale.data_ptr(), bptr,
@@ -709,7 +699,7 @@ at::Tensor w4_linear_hip(const at::Tensor& input, const at::Tensor& weight, cons
   const void* bptr = (bias.has_value() && bias->defined()) ? bias->data_ptr() : nullptr;
   const rf_w8a16_proj proj{weight.data_ptr(), sc.data_ptr(), bptr, y.data_ptr(), N, N};
   const int st = with_scratch(
-      x2.device(), stream, M, op,
+      x2.device(), stream, op,
       [&](const rf_w8a16_scratch* scratch) {
         return rf_w4a16_linear_multi_scratch(x2.data_ptr(), x2.stride(0), &proj, 1,
                                              (int32_t)group_size, M, K, (int32_t)kernel, scratch,
@@ -796,7 +786,7 @@ std::vector<at::Tensor> w4_linear_multi_hip(const at::Tensor& input, at::TensorL
   c10::DeviceGuard dev_guard(x2.device());
   void* stream = c10::hip::getCurrentHIPStream(x2.device().index()).stream();
   const int st = with_scratch(
-      x2.device(), stream, M, op,
+      x2.device(), stream, op,
       [&](const rf_w8a16_scratch* scratch) {
         return rf_w4a16_linear_multi_scratch(x2.data_ptr(), x2.stride(0), projs, (int32_t)count,
                                              (int32_t)group_size, M, K, (int32_t)kernel, scratch,

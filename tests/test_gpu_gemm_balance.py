@@ -178,18 +178,19 @@ def test_last_tiles_of_a_launch_beyond_the_counters():
 
 @pytest.mark.gpu
 def test_last_tiles_under_capture():
-    """A capture does not grow the stream's workspace for the split of the last
-    tiles: it runs them whole, and an eager call before the first replay finds
-    cleared counters."""
+    """A capture on a stream whose scratch is still at its least size splits the
+    last tiles as an eager call does: the same bits in both, whatever ran on the
+    stream before, and counters that eager calls find cleared."""
     m, n, k = 1300, 24576, 3072
     print(f"last tiles under capture M={m} N={n} K={k}", flush=True)
     x, q, s = _big(m, n, k)
     packed = rf.pack_weight(q)
     split, whole = rf.linear(x, packed, s), _unsplit(x, packed, s, n)
+    assert not torch.equal(split, whole)  # (the comparison below would see the other order)
     stream = torch.cuda.Stream()
     stream.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(stream):
-        rf.linear(x[:1], packed, s)  # the stream's workspace at its least size
+        rf.linear(x[:1], packed, s)  # the stream's scratch at its least size
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=stream):
         y = rf.linear(x, packed, s)
@@ -202,7 +203,7 @@ def test_last_tiles_under_capture():
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(y, whole)
+        assert torch.equal(y, split)
         assert torch.equal(rf.linear(x, packed, s), split)
 
 
