@@ -331,16 +331,23 @@ hipError_t launch_quant_t(const QuantArgs& a, int layout, hipStream_t stream) {
 template <int VEC>
 hipError_t launch_embed_t(const int8_t* table, int64_t V, int64_t H, const _Float16* scale,
                           const void* ids, bool ids64, int64_t M, _Float16* y, hipStream_t stream) {
+  // A launch holds fewer than 2^32 threads along x, so fewer than 2^24
+  // workgroups of 256; more rows than that take several launches.
   const int64_t per_row = ceil_div(H, 256 * VEC);
-  if (M * per_row > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(M * per_row));
-  if (ids64)
-    hipLaunchKernelGGL((embed_kernel<VEC, int64_t>), grid, dim3(256), 0, stream, table, V, H, scale,
-                       static_cast<const int64_t*>(ids), (int)per_row, y);
-  else
-    hipLaunchKernelGGL((embed_kernel<VEC, int32_t>), grid, dim3(256), 0, stream, table, V, H, scale,
-                       static_cast<const int32_t*>(ids), (int)per_row, y);
-  return hipGetLastError();
+  const int64_t rows = (((int64_t)1 << 24) - 1) / per_row;
+  if (rows < 1) return hipErrorInvalidValue;
+  for (int64_t m0 = 0; m0 < M; m0 += rows) {
+    const dim3 grid((unsigned)((M - m0 < rows ? M - m0 : rows) * per_row));
+    if (ids64)
+      hipLaunchKernelGGL((embed_kernel<VEC, int64_t>), grid, dim3(256), 0, stream, table, V, H, scale,
+                         static_cast<const int64_t*>(ids) + m0, (int)per_row, y + m0 * H);
+    else
+      hipLaunchKernelGGL((embed_kernel<VEC, int32_t>), grid, dim3(256), 0, stream, table, V, H, scale,
+                         static_cast<const int32_t*>(ids) + m0, (int)per_row, y + m0 * H);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 bool aligned_to(const void* p, size_t n) { return (uintptr_t)p % n == 0; }

@@ -879,6 +879,8 @@ at::Tensor embedding_eager(const at::Tensor& weight, const at::Tensor& scale,
   return (rows * at::index(scale, idx).to(at::kFloat).unsqueeze(-1)).to(at::kHalf);
 }
 
+constexpr int64_t kMaxRows = (int64_t)1 << 30;  // the C ABI's bound on every size
+
 bool int_ids(const at::Tensor& ids) {
   return ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt;
 }
@@ -890,8 +892,8 @@ at::Tensor embedding_hip(const at::Tensor& weight, const at::Tensor& scale, cons
                       scale.size(0) == weight.size(0) && weight.is_contiguous() &&
                       scale.is_contiguous() && weight.numel() > 0 && ids.numel() > 0 &&
                       ids.device() == weight.device() && scale.device() == weight.device() &&
-                      // (the launch grid: one workgroup per 256 values at the narrowest)
-                      ids.numel() * ceil_div(weight.size(1), 256) <= 0x7fffffff;
+                      ids.numel() <= kMaxRows && weight.size(0) <= kMaxRows &&
+                      weight.size(1) <= kMaxRows;
   if (!kernel) return embedding_eager(weight, scale, ids);
   const int64_t V = weight.size(0), H = weight.size(1), M = ids.numel();
   const at::Tensor i = ids.contiguous();

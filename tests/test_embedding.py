@@ -75,3 +75,19 @@ def test_gpu_forms(v, h):
     assert torch.equal(emb(ids), _want(q, s, ids))
     strided = torch.as_strided(ids, (35, 3), (2, 70))
     assert torch.equal(emb(strided), _want(q, s, strided))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,h", [((1 << 24) + 5, 16), ((1 << 23) + 3, 257)])
+def test_gpu_more_rows_than_one_launch_holds(m, h):
+    """A launch holds fewer than 2^24 workgroups of 256 threads, one (16-wide
+    rows) or two (257-wide, a value per thread) to a row here."""
+    print(f"embedding of {m} ids x {h}", flush=True)
+    q, s = _table(1000, h, "cuda")
+    for dtype in (torch.int64, torch.int32):
+        ids = torch.randint(-1000, 1000, (m,), device="cuda", dtype=dtype)
+        got = rf.W8A16Embedding(q, s)(ids)
+        for i in range(0, m, 1 << 20):
+            part = ids[i:i + (1 << 20)]
+            assert torch.equal(got[i:i + (1 << 20)], _want(q, s, part)), i
+        del got
