@@ -327,7 +327,14 @@ class W8A16Embedding(nn.Module):
         self.register_buffer("weight_scale", weight_scale.contiguous())
 
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
+        if not isinstance(input_ids, torch.Tensor):  # a list, an int, a slice
+            return self._index(input_ids)
         return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
+
+    def _index(self, ids):
+        """The lookup in torch operations, for whatever torch indexing takes."""
+        rows = self.weight[ids].to(torch.float32)
+        return (rows * self.weight_scale[ids].to(torch.float32).unsqueeze(-1)).to(torch.float16)
 
     def extra_repr(self) -> str:
         return f"{self.num_embeddings}, {self.embedding_dim}, int8 rows"

@@ -3,6 +3,7 @@ the CPU and under meta / vmap / autograd, against the torch expression; the HIP
 kernel (16-, 8- and 1-wide) byte for byte against the same on the GPU."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -44,6 +45,26 @@ def test_cpu_forms():
         rf.W8A16Embedding(q, s)(torch.tensor([50]))
     with pytest.raises(IndexError):
         rf.W8A16Embedding(q, s)(torch.tensor([0.5]))
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_indices_that_are_not_tensors(dev):
+    q, s = _table(50, 24, dev)
+    emb = rf.W8A16Embedding(q, s)
+    for ids in (7, -1, [3, 1, -50], slice(2, 9), np.array([[4, 5]]), ([1, 2],), ...):
+        assert torch.equal(emb(ids), _want(q, s, ids)), ids
+    with pytest.raises(IndexError):
+        emb(50)
+
+
+def test_scripted_and_traced():
+    q, s = _table(50, 24)
+    emb = rf.W8A16Embedding(q, s)
+    ids = torch.tensor([[3, 1], [-1, 7]])
+    for m in (torch.jit.script(emb), torch.jit.trace(emb, ids),
+              torch.export.export(emb, (ids,)).module(),
+              torch.compile(emb, backend="eager", fullgraph=True)):
+        assert torch.equal(m(ids), _want(q, s, ids))
 
 
 def test_transforms():
