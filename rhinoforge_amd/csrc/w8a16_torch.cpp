@@ -1033,7 +1033,10 @@ TORCH_LIBRARY_IMPL(rhinoforge, CUDA, m) {
   m.impl("quantize_pack", TORCH_FN(quantize_pack));
   m.impl("embedding", TORCH_FN(embedding_hip));
 }
-TORCH_LIBRARY_IMPL(rhinoforge, CPU, m) { m.impl("embedding", TORCH_FN(embedding_eager)); }
+// (any other device, the CPU among them)
+TORCH_LIBRARY_IMPL(rhinoforge, CompositeExplicitAutograd, m) {
+  m.impl("embedding", TORCH_FN(embedding_eager));
+}
 TORCH_LIBRARY_IMPL(rhinoforge, FuncTorchBatched, m) { m.impl("embedding", TORCH_FN(embedding_eager)); }
 TORCH_LIBRARY_IMPL(rhinoforge, Meta, m) {
   m.impl("embedding", TORCH_FN(embedding_meta));

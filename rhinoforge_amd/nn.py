@@ -302,6 +302,9 @@ class W4A16Linear(_LogicalWeightStateDict, nn.Module):
                 f"bias={self.bias is not None}, {mode}, layout=TILE16X128_I4")
 
 
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
 class W8A16Embedding(nn.Module):
     """Token embedding with an int8 row-major table and one fp16 scale per row.
 
@@ -327,9 +330,15 @@ class W8A16Embedding(nn.Module):
         self.register_buffer("weight_scale", weight_scale.contiguous())
 
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
-        if not isinstance(input_ids, torch.Tensor):  # a list, an int, a slice
-            return self._index(input_ids)
-        return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
+        if torch.jit.is_scripting():
+            return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
+        weight, scale = self.weight, self.weight_scale
+        # The op takes plain tensors.  A list, an int or a slice is indexed with
+        # as torch does, and a tensor subclass (DTensor, FakeTensor) brings its
+        # own indexing along, while it knows nothing of the op.
+        if (type(input_ids) is torch.Tensor and type(weight) in _PLAIN and type(scale) in _PLAIN):
+            return torch.ops.rhinoforge.embedding(weight, scale, input_ids)
+        return self._index(input_ids)
 
     def _index(self, ids):
         """The lookup in torch operations, for whatever torch indexing takes."""

@@ -67,6 +67,28 @@ def test_scripted_and_traced():
         assert torch.equal(m(ids), _want(q, s, ids))
 
 
+def test_tensor_subclasses(tmp_path):
+    """Sharded tables and ids, and fake tensors, through their own indexing."""
+    import torch.distributed as dist
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.distributed.tensor import Replicate, Shard, distribute_tensor, init_device_mesh
+    q, s = _table(50, 24)
+    ids = torch.tensor([[3, 1], [-1, 7]])
+    with FakeTensorMode() as mode:
+        y = rf.W8A16Embedding(mode.from_tensor(q), mode.from_tensor(s))(mode.from_tensor(ids))
+        assert y.shape == (2, 2, 24) and y.dtype == torch.float16
+    dist.init_process_group("gloo", init_method=f"file://{tmp_path}/store", rank=0, world_size=1)
+    try:
+        mesh = init_device_mesh("cpu", (1,))
+        di = distribute_tensor(ids, mesh, [Replicate()])
+        for place in (Replicate(), Shard(0), Shard(1)):
+            emb = rf.W8A16Embedding(distribute_tensor(q, mesh, [place]),
+                                    distribute_tensor(s, mesh, [Replicate()]))
+            assert torch.equal(emb(di).full_tensor(), _want(q, s, ids)), place
+    finally:
+        dist.destroy_process_group()
+
+
 def test_transforms():
     q, s = _table(50, 24)
     ids = torch.tensor([[3, 1], [-1, 7]])
