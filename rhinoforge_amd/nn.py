@@ -160,6 +160,9 @@ class W8A16Linear(_LogicalWeightStateDict, nn.Module):
         in one kernel, without the row-major values in between)."""
         w = linear.weight.detach()
         if on_kernel(w):
+            if linear.bias is not None and tuple(linear.bias.shape) != (w.size(0),):
+                raise ValueError(f"bias must have shape ({w.size(0)},), got "
+                                 f"{tuple(linear.bias.shape)}")
             mod = cls(w.size(1), w.size(0), bias=linear.bias is not None, device="meta")
             mod.weight, mod.weight_scale = torch.ops.rhinoforge.quantize_pack(w, 8, 0)
             if linear.bias is not None:

@@ -129,3 +129,13 @@ def test_modules_from_linear():
         for name in ("weight", "weight_scale", "bias"):
             _same(getattr(m, name), getattr(ref, name))
         assert (m.in_features, m.out_features) == (1088, 48)
+
+
+def test_from_linear_refuses_a_bias_of_another_shape():
+    """As on the CPU: refused when the module is made, not by its first call."""
+    for dev in ("cpu", DEV):
+        for shape in ((47,), (1, 48), ()):
+            lin = torch.nn.Linear(64, 48, device=dev)
+            lin.bias = torch.nn.Parameter(torch.zeros(shape, device=dev))
+            with pytest.raises(ValueError, match="bias must have shape"):
+                rf.W8A16Linear.from_linear(lin)
