@@ -133,8 +133,7 @@ int rf_w8a16_quantize_device(const void* w, int32_t dtype, int64_t N, int64_t K,
  * f32(scale[id])) for id = ids[m] (python/rpu_backend/adapters/qwen3.py:654-680).
  *   table : int8 [V,H] row-major;  scale : fp16 [V];  y : fp16 [M,H]
  *   ids   : int64 (ids64 != 0) or int32 [M], in [-V, V) (negative ids count
- *           from the end); an id outside aborts the kernel, so the stream's
- *           next synchronization reports an error. */
+ *           from the end); an id outside gives a row of NaN. */
 int rf_w8a16_embedding(const void* table, int64_t V, int64_t H, const void* scale,
                        const void* ids, int32_t ids64, int64_t M, void* y, void* stream);
 

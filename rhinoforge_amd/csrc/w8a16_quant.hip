@@ -269,9 +269,11 @@ __global__ __launch_bounds__(256) void embed_kernel(const int8_t* __restrict__ t
   const int64_t h = ((int64_t)(blockIdx.x - (uint32_t)m * (uint32_t)per_row) * 256 + threadIdx.x) * VEC;
   int64_t id = (int64_t)ids[m];
   if (id < 0) id += V;  // as torch indexing counts from the end
-  if ((uint64_t)id >= (uint64_t)V) __builtin_trap();  // an index out of range is an error
+  // An id outside the table gives a row of NaN (a trap would end the process).
+  const bool inside = (uint64_t)id < (uint64_t)V;
+  if (!inside) id = 0;
   if (h >= H) return;
-  const float s = (float)scale[id];
+  const float s = inside ? (float)scale[id] : __builtin_nanf("");
   const int8_t* q = table + id * H + h;
   _Float16* o = y + m * H + h;
   if constexpr (VEC == 1) {

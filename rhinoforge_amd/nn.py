@@ -315,7 +315,9 @@ class W8A16Embedding(nn.Module):
     343-356): ``weight`` int8 [V, H], ``weight_scale`` fp16 [V].  A lookup
     gathers rows and dequantizes them as ``fp16(f32(q) * f32(s))``
     (adapters/qwen3.py:654-680), in one kernel on a HIP device; the table is
-    gathered, never multiplied, so it stays row-major.
+    gathered, never multiplied, so it stays row-major.  An id outside the table
+    raises IndexError on the CPU; on a HIP device, where the call does not wait
+    for the ids, it gives a row of NaN.
     """
 
     def __init__(self, weight: torch.Tensor, weight_scale: torch.Tensor,

@@ -134,3 +134,18 @@ def test_gpu_more_rows_than_one_launch_holds(m, h):
             part = ids[i:i + (1 << 20)]
             assert torch.equal(got[i:i + (1 << 20)], _want(q, s, part)), i
         del got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h", [4096, 24, 7])
+def test_gpu_ids_outside_the_table(h):
+    """Rows of NaN, without a read outside the table; the other rows as always."""
+    print(f"embedding ids outside the table, width {h}", flush=True)
+    v = 50
+    q, s = _table(v, h, "cuda")
+    bad = [v, -v - 1, 2**31 - 1, -2**31, 2**40, -2**62]
+    for dtype, n in ((torch.int64, 6), (torch.int32, 4)):
+        ids = torch.tensor([3, *bad[:n], -1], device="cuda", dtype=dtype)
+        y = rf.W8A16Embedding(q, s)(ids)
+        assert y[1:-1].isnan().all()
+        assert torch.equal(y[[0, -1]], _want(q, s, ids[[0, -1]]))
