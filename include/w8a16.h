@@ -124,7 +124,9 @@ int rf_w8a16_pack_weight_device(const int8_t* q_dev, int64_t N, int64_t K,
  *   layout ROWMAJOR     q int8 [N,K] row-major (N*K bytes)
  *   layout TILE16X64    (bits 8, group_size 0) as rf_w8a16_pack_weight of those values
  *   layout TILE16X128_I4 (bits 4) as rf_w4a16_pack_weight of those values
- * scale is 2-byte, packed output 16-byte aligned; w aligned to its type. */
+ * scale is 2-byte, packed output 16-byte aligned; w aligned to its type.  One
+ * launch holds N < 2^26 - 16 rows and, with groups, K < 2^26 - 1024 columns;
+ * larger matrices: RF_W8A16_EHIP. */
 int rf_w8a16_quantize_device(const void* w, int32_t dtype, int64_t N, int64_t K, int64_t ldw,
                              int32_t bits, int32_t group_size, int32_t layout, void* q,
                              size_t q_bytes, void* scale, void* stream);

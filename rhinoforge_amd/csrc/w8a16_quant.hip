@@ -305,7 +305,7 @@ template <int DT>
 hipError_t launch_quant_t(const QuantArgs& a, int layout, hipStream_t stream) {
   const dim3 block(256);
   const int64_t gx = ceil_div(a.rows, 4);
-  if (gx > 0x7fffffff) return hipErrorInvalidValue;
+  if (gx >= (int64_t)1 << 24) return hipErrorInvalidValue;  // (fewer than 2^32 threads along x)
   if (a.group) {
     const int64_t gy = ceil_div(a.chunks, 64);
     if (gy > 65535) return hipErrorInvalidValue;

@@ -41,15 +41,17 @@ def round_to_levels(w32: torch.Tensor, step16: torch.Tensor, lo: int, hi: int) -
 
 
 _KERNEL_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+_KERNEL_SIZE = 2**26 - 1024  # rows (four to a workgroup) and columns one launch holds
 
 
 def on_kernel(weight: torch.Tensor) -> bool:
     """Whether the device quantizer takes this matrix: a plain HIP tensor (or
-    parameter) of a type it reads, non-empty, outside functorch transforms and
-    forward-mode AD.  Everything else keeps the torch arithmetic below, which
+    parameter) of a type it reads, non-empty, of sizes one launch holds, outside
+    functorch transforms and forward-mode AD.  Everything else keeps the torch arithmetic below, which
     gives the same bytes."""
     return (type(weight) in (torch.Tensor, torch.nn.Parameter) and weight.is_cuda
             and weight.dim() == 2 and weight.dtype in _KERNEL_DTYPES and weight.numel() > 0
+            and weight.size(0) < _KERNEL_SIZE and weight.size(1) < _KERNEL_SIZE
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0)
 

@@ -139,3 +139,23 @@ def test_from_linear_refuses_a_bias_of_another_shape():
             lin.bias = torch.nn.Parameter(torch.zeros(shape, device=dev))
             with pytest.raises(ValueError, match="bias must have shape"):
                 rf.W8A16Linear.from_linear(lin)
+
+
+def test_more_rows_than_one_launch_holds():
+    """2^26 rows of one repeated pattern: the torch arithmetic, as on the CPU."""
+    n, k = 2**26, 8
+    w = torch.tensor([0.5, -1, 0.25, 0, 1.5, -2, 3, 1], device=DEV, dtype=torch.float16)
+    q, s = rf.quantize_linear_per_channel(w.expand(n, k))
+    q1, s1 = rf.quantize_linear_per_channel(w.expand(1, k).cpu())
+    assert q.shape == (n, k) and bool((q == q1.to(DEV)).all()) and bool((s == s1.to(DEV)).all())
+    edge = w.expand(_common._KERNEL_SIZE - 1, k)     # the most the kernel takes
+    assert _common.on_kernel(edge)
+    q, s = rf.quantize_linear_per_channel(edge)
+    assert bool((q == q1.to(DEV)).all()) and bool((s == s1.to(DEV)).all())
+    x = torch.zeros(1, 2**26, device=DEV, dtype=torch.float16)
+    x[0, ::32] = 7.0
+    q, s, _ = rf.quantize_int4_group_wise(x, 32)
+    assert s.shape == (2**21, 1) and bool((s == 1).all()) and int(q.sum()) == 7 * 2**21
+    x = x[:, :_common._KERNEL_SIZE - 32]
+    q, s, _ = rf.quantize_int4_group_wise(x, 32)
+    assert bool((s == 1).all()) and int(q.sum()) == 7 * (x.size(1) // 32)
