@@ -1156,12 +1156,15 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
     if (one_row && (many ? c.cfg == kV3M128N128KG
                          : c.cfg != kV3M64N64KG || 4 * tiles > cus)) continue;
     for (int s = 1; s <= 4; ++s) {
-      // (three splits only where four of the 128-wide forms do not fit one
-      // round, and at M > 128 only from K 4545 on: shorter launches keep
-      // the 64x64 plan that test_linear_multi_two_k_groups holds them to,
-      // although three splits are ahead there too: 2560 x 4096 at M 256 14.6
-      // instead of 16.3 us)
-      if (s == 3 && (c.cfg == kV3M64N64KG || 4 * tiles <= cus || (M > 128 && kblocks < 72))) continue;
+      // Three splits only where four of the 128-wide forms do not fit one
+      // round, and at M > 128 from 64 K blocks on.  There they are ahead of the
+      // unsplit smaller tile and of four splits of 128x128 (MI355X, graph-timed,
+      // rotated weights, 122 launches of M 129..512, K 3072..4544 whose plan it
+      // decides: 0.75..1.008 of the time from K 4096 on, 2560 x 4096 at M 256
+      // 17.0 -> 15.0 us, 5120 x 4096 23.7 -> 22.2, 1536 x 4544 at M 384 19.5 ->
+      // 15.7), while shorter splits lose to the hand-off (K 3072..3840 up to
+      // 1.12: 3584 x 3080 at M 384 19.5 -> 21.8).
+      if (s == 3 && (c.cfg == kV3M64N64KG || 4 * tiles <= cus || (M > 128 && kblocks < 64))) continue;
       if (tiles * s > cus || kblocks < 16 * s || (s > 1 && tiles > kMaxSplitTiles)) continue;
       if (beyond && (s > 2 || 4 * tiles * s < 3LL * cus)) continue;
       const int kbs = (int)ceil_div(kblocks, s);

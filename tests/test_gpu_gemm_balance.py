@@ -26,6 +26,10 @@ ROWS = [
     # M 65 and more: three splits of a 128-wide form where four do not fit
     (250, [5000], 8200, "gemm 128x128 two K groups", 3),
     (100, [5112], 4104, "gemm 64x128 two K groups", 3),
+    # ... at M > 128 from 64 K blocks on
+    (256, [1000, 520, 520], 4104, "gemm 64x128 two K groups", 3),
+    (250, [5000], 4040, "gemm 128x128 two K groups", 3),
+    (250, [5000], 4032, "gemm 64x128 two K groups", 1),
 ]
 
 # int4 launches of large tiles: (M, N per projection, K, group size, plan, splits)
