@@ -821,7 +821,8 @@ hipError_t launch_t(const GemvKernelArgs& ka, const GemvPlan& p, hipStream_t str
   return hipGetLastError();
 }
 
-// The one-strip configurations without an x copy: x through wavefront-private
+// The one-strip configurations without an x copy (int4: the 16-wavefront one;
+// the others are planned up to M = 4 only): x through wavefront-private
 // tiles from M = 9, and for int4, whose x tile is four times its weight tile,
 // from M = 5 where a wavefront has more than one tile (with one, 3072 x 1024 at
 // M 5, 3% slower).  There every fragment serves one weight tile only; with three
@@ -978,12 +979,12 @@ hipError_t launch_gemv4_cfg(const GemvKernelArgs& ka, const GemvPlan& p, hipStre
         if (WF == kWfInt4) return launch_t<1, 1, 16, 2, true, true, WF>(ka, p, stream);
         return launch_t<1, 1, 16, 1, true, true, WF>(ka, p, stream);
       }
-      return launch_1<16, 1, WF>(ka, p, stream);
+      return launch_t<1, 1, 16, 1, false, true, WF>(ka, p, stream);
     case kG1x1W8U4XL:
       if (xl_fits(1, 8)) return launch_t<1, 1, 8, 2, true, true, WF>(ka, p, stream);
-      return launch_1<8, 2, WF>(ka, p, stream);
+      return launch_t<1, 1, 8, 2, false, true, WF>(ka, p, stream);
     case kG1x1W16U2: return launch_1<16, 1, WF>(ka, p, stream);
-    case kG1x1W8U4: return launch_1<8, 2, WF>(ka, p, stream);
+    case kG1x1W8U4: return launch_t<1, 1, 8, 2, false, true, WF>(ka, p, stream);
     case kG1x1W4U4: return launch_t<1, 1, 4, 2, false, true, WF>(ka, p, stream);
     case kG1x2W16U2: return launch_t<1, 2, 16, 1, false, true, WF>(ka, p, stream);
     case kG1x4W8U2: return launch_t<1, 4, 8, 1, false, true, WF>(ka, p, stream);
