@@ -1127,18 +1127,24 @@ static bool plan_two_k_groups(int M, const int* Ns, int nproj, int K, int cus, i
   if (beyond && kblocks > 80) return false;
   // At M 33..64 on <= 64 tiles of 64x64 only that form with four K splits
   // (K >= 4096): -8..-14% against the 64x64 4-stage tile with 8 splits at
-  // N 1024..4096, K 4096..8192; at N 5120 / 8192 mixed (-7..+4%).  From 96
-  // tiles (N >= 6144 in all) and K 2048 on, the 64x128 and 64x64 forms by the
+  // N 1024..4096, K 4096..8192.  On more tiles the 64x128 and 64x64 forms by the
   // estimate below: one round of workgroups that each fill a CU, where 64x64
-  // tiles with four to eight splits left CUs with one or two more than others
-  // (M 41: Qwen3-VL-32B q/k/v, three splits of 64x128, 17.9 instead of 21.3
-  // us; 19456 x 2560 17.7 instead of 21.8; 12288 x 2048 11.6 instead of 13.7).
+  // tiles with four to eight splits left CUs with one or two more than others.
+  // From 96 tiles (N >= 6144 in all) that is ahead from K 2048 on (M 41:
+  // Qwen3-VL-32B q/k/v, three splits of 64x128, 17.9 instead of 21.3 us; 19456
+  // x 2560 17.7 instead of 21.8; 12288 x 2048 11.6 instead of 13.7); on 65..95
+  // tiles from 46 K blocks, where the estimate takes two splits and more, up to
+  // 128 (MI355X, graph-timed, rotated weights, 160 launches of M 33..64, N
+  // 4161..6017, K 2952..8192: 0.83..1.00 of the time, 0.92 in the mean; 4608 x
+  // 3584 at M 41 13.1 -> 12.3 us, 4224 x 4096 at M 64 16.5 -> 13.7).  Unsplit
+  // at K 2560 / 2816 it is 1.09 at the worst, beyond K 8192 up to 1.04 at M 33.
   const bool one_row = M <= 64;
   bool many = false;
   if (one_row) {
     int64_t t64 = 0;
     for (int i = 0; i < nproj; ++i) t64 += ceil_div(Ns[i], 64);
-    many = 8 * t64 >= 3LL * cus && kblocks >= 32;
+    many = 8 * t64 >= 3LL * cus ? kblocks >= 32
+                                : 4 * t64 > cus && kblocks >= 46 && kblocks <= 128;
     if (!many && kblocks < 64) return false;
   }
   struct Cand {

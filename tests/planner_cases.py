@@ -347,7 +347,12 @@ GEMM_POLICY = [
     (48, 1024, 4096, "gemm 64x64 two K groups", 64, 64, 4),
     (33, 1000, 4104, "gemm 64x64 two K groups", 64, 64, 4),  # ragged N and K
     (64, 4096, 8192, "gemm 64x64 two K groups", 64, 64, 4),
-    (48, 5120, 4096, "gemm 64x64 4-stage", 64, 64, 8),  # 80 tiles: more than 64
+    # M 33..64, 65..95 tiles of 64x64, 46..128 K blocks: two K groups by the estimate
+    (41, 4608, 3584, "gemm 64x64 two K groups", 64, 64, 2),  # 72 tiles
+    (33, 4161, 2888, "gemm 64x64 two K groups", 64, 64, 2),  # 66 tiles, 46 K blocks, ragged
+    (48, 5120, 4096, "gemm 64x128 two K groups", 64, 128, 4),  # 80 tiles
+    (64, 6020, 8192, "gemm 64x128 two K groups", 64, 128, 4),  # 95 tiles, 128 K blocks
+    (48, 5120, 2880, "gemm 64x64 4-stage", 64, 64, 4),  # 80 tiles, 45 K blocks
     (64, 2048, 2048, "gemm 64x64 4-stage", 64, 64, 4),  # K < 4096
     # M 65..127 with few tiles: two K groups
     (100, 520, 1032, "gemm 64x64 two K groups", 64, 64, 1),
@@ -391,7 +396,7 @@ GEMM_POLICY = [
     # M = 1 forced to the GEMM: 16 tiles of 32x64, 4-way split
     (1, 1024, 4096, "gemm 32x64 3-stage", 32, 64, 4),
     # M 33..64: 64x64 tiles, split to ~3 workgroups per CU
-    (48, 5120, 8192, "gemm 64x64 4-stage", 64, 64, 8),     # 80 tiles, 8-way split
+    (48, 5120, 8200, "gemm 64x64 4-stage", 64, 64, 8),     # 80 tiles, 8-way split, 129 K blocks
     # M 33..64, 100 tiles of 64x256 (>= 96): 64x256 with a 2-way K split
     (40, 25600, 5120, "gemm 64x256 3-stage", 64, 256, 2),
     # M 33..64, 193 tiles of 64x256 (>= 192): 64x256, no split; ragged N, K tail
