@@ -337,11 +337,17 @@ class W8A16Embedding(nn.Module):
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
         if torch.jit.is_scripting():
             return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
-        weight, scale = self.weight, self.weight_scale
+        # (read from the buffers themselves: nn.Module's attribute lookup costs
+        # 0.3 us of a 7 us call each; attributes where they are no longer
+        # buffers, as under a parametrization)
+        buffers = self._buffers
+        weight, scale = buffers.get("weight"), buffers.get("weight_scale")
+        if weight is None or scale is None:
+            weight, scale = self.weight, self.weight_scale
         # The op takes plain tensors.  A list, an int or a slice is indexed with
         # as torch does, and a tensor subclass (DTensor, FakeTensor) brings its
         # own indexing along, while it knows nothing of the op.
-        if (type(input_ids) is torch.Tensor and type(weight) in _PLAIN and type(scale) in _PLAIN):
+        if type(input_ids) is torch.Tensor and type(weight) in _PLAIN and type(scale) in _PLAIN:
             return torch.ops.rhinoforge.embedding(weight, scale, input_ids)
         return self._index(input_ids)
 

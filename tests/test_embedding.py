@@ -104,6 +104,30 @@ def test_transforms():
     assert m.shape == (2, 2, 24) and m.dtype == torch.float16
 
 
+def test_replaced_buffers():
+    """The lookup reads what the module holds: another tensor, a parameter in the
+    buffer's place, a parametrization, functional_call's tensors."""
+    from torch.nn.utils import parametrize
+    q, s = _table(50, 24)
+    ids = torch.tensor([[3, 1], [-1, 7]])
+
+    class Halve(torch.nn.Module):
+        def forward(self, t):
+            return t * 0.5
+
+    emb = rf.W8A16Embedding(q, s)
+    emb.weight = q.flip(0).contiguous()
+    assert torch.equal(emb(ids), _want(q.flip(0), s, ids))
+    swap = {"weight": q, "weight_scale": s * 2}
+    assert torch.equal(torch.func.functional_call(emb, swap, (ids,)), _want(q, s * 2, ids))
+    parametrize.register_parametrization(emb, "weight_scale", Halve())
+    assert torch.equal(emb(ids), _want(q.flip(0), s * 0.5, ids))
+    emb = rf.W8A16Embedding(q, s)
+    del emb.weight_scale
+    emb.weight_scale = torch.nn.Parameter(s * 4)
+    assert torch.equal(emb(ids), _want(q, s * 4, ids))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("v,h", [(300, 4096), (97, 4112), (50, 24), (33, 8), (20, 7), (9, 1),
                                  (1000, 5120)])
