@@ -152,8 +152,9 @@ __device__ __forceinline__ void store_chunk(const QuantArgs& a, int64_t n, int c
 // amax and the rounding pass (rows up to 4096 wide are read from memory once),
 // the rest are read again, from the caches.  A chunk of a tile layout is one
 // 16-byte store; four rows fill 64 contiguous bytes of a tile.
-// (12288 x 4096 bf16 -> TILE16X64: 30 us, the time of a device copy of the
-// input; 636 us as ten elementwise passes, a reduction and the pack kernel.)
+// (12288 x 4096 bf16 -> TILE16X64: 31 us, 4.9 TB/s over the 151 MB it reads and
+// writes, the rate of a large device copy; 636 us the call as ten elementwise
+// passes, a reduction and the pack kernel.)
 constexpr int kKeep = 4;
 template <int DT, int LAYOUT>
 __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
