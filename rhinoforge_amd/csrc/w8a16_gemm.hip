@@ -1250,19 +1250,24 @@ static bool plan_long_k_two_groups(int M, const int* Ns, int nproj, int K, int c
 }
 
 // Packed int4 at M <= 64 and on launches of few 128x128 tiles (t128) beyond:
-// the tiles of 128-wide K blocks.  These launches are bound by instruction
-// issue, not by memory (with every load aimed at cached lines they take the
-// same time): a stage is about 52 VALU operations per strip to dequantize plus
-// the MFMAs, and a CU with two workgroups does more of them per microsecond
-// than with one.  So the plan takes the least estimated time over the tiles
-// and 1..8 K splits of
+// the tiles of 128-wide K blocks.  These launches are bound by latency: the
+// wait for a stage, the barrier and the LDS reads stand before each block's
+// dequantization, and a wavefront waits for 40..55% of its cycles, while the
+// VALUs are busy for 20..37% and the MFMA pipes for 9..18% of the CUs' busy
+// cycles (counters of a 4B gs 128 layer at M 48).  A CU with two workgroups
+// fills one's waits with the other's work and does more per microsecond than
+// with one.  So the plan takes the least estimated time over the tiles and
+// 1..8 K splits of
 //   2.2 + 1.1 c + blocks * (c == 1 ? alone : c * shared) + hand-off us,
 // with c workgroups on the fullest CU, `blocks` 128-wide K blocks per
 // workgroup, the tile's time per block alone on a CU and when it shares one,
 // and a hand-off of 1.2 us + 0.4 us per split and 4096 outputs of the tile.
-// The constants are a least-squares fit to 11600 timed launches (MI355X, N
-// 512..37888, K 1024..25600, M 17..512, per-channel, gs 32 and 128; rms error
-// 8%); over those shapes its choice is 1.3..3% off the best one at M <= 128.
+// The constants are a least-squares fit to timed launches.  On 2323 others
+// (MI355X, 120 random shapes of M 17..512, N 512..37888, K 1024..25600,
+// per-channel, gs 32 and 128, every tile and split; profiles/int4_plan_fit.md)
+// the estimate is 0.5% high in the mean with an rms error of 10% (per-channel
+// 7% high, group-wise 4% low), and the tile and split it takes 2.5% off the
+// best at M <= 64, 1.4% up to M 128, 1.1% beyond, 13% at the worst.
 // Against the plans before (the GEMV up to M 64, 64x256 and 128-row tiles
 // beyond): 0.61 of the time at M 33..64 (19456 x 2560 at M 48 28.9 -> 15.9
 // us, 5120 x 25600 68.3 -> 29.4), 0.70 at M 65..128 (1024 x 2048 at M 96 16.6
