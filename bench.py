@@ -516,8 +516,10 @@ def bench_cfg2(torch, rf):
 
 def bench_cfg4(torch, rf):
     """cfg4: Qwen3-VL-32B projections at M in {1, 32, 512}, four layer copies
-    (1.96 GB): every projection's copies together exceed the 256 MB Infinity
-    Cache.  M 1 and 32 are judged against HBM, M 512 against MFMA."""
+    (1.96 GB).  The copies of gate, up, down and gate/up (0.5..1 GB each) exceed
+    the 256 MB Infinity Cache; those of q, o (168 MB), k, v (21 MB) and the fused
+    q/k/v (210 MB) fit in it, and their rows are times of weights that may come
+    from there.  M 1 and 32 are judged against HBM, M 512 against MFMA."""
     copies = [make_layer(torch, rf, QWEN3_VL_32B, seed=940 + c) for c in range(4)]
     rows = []
     for m in (1, 32, 512):
@@ -660,7 +662,9 @@ def nbytes_w4(m, n, k, gs):
 def bench_w4a16(torch, rf):
     """W4A16 on the same Qwen3-8B shapes: decode projections at M 1 and 16 and the
     M=2048 MLP prefill, per-channel and group-wise (32, 128); random int4 values
-    and scales, four rotated layer copies (384 MB, past the Infinity Cache)."""
+    and scales, four rotated layer copies (384 MB).  The layer of four launches
+    rotates them all, past the 256 MB Infinity Cache; the copies of a single
+    projection (8..101 MB) fit in it."""
     rows = []
     for gs in (0, 32, 128):
         copies = []
