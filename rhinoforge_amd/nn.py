@@ -337,9 +337,9 @@ class W8A16Embedding(nn.Module):
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
         if torch.jit.is_scripting():
             return torch.ops.rhinoforge.embedding(self.weight, self.weight_scale, input_ids)
-        # (read from the buffers themselves: nn.Module's attribute lookup costs
-        # 0.3 us of a 7 us call each; attributes where they are no longer
-        # buffers, as under a parametrization)
+        # (read from the buffers themselves: as attributes, through nn.Module's
+        # lookup, a call takes 6.7 us instead of 6.2; attributes where they are
+        # no longer buffers, as under a parametrization)
         buffers = self._buffers
         weight, scale = buffers.get("weight"), buffers.get("weight_scale")
         if weight is None or scale is None:
