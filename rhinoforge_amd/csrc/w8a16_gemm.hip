@@ -1264,7 +1264,7 @@ static bool plan_long_k_two_groups(int M, const int* Ns, int nproj, int K, int c
 // and a hand-off of 1.2 us + 0.4 us per split and 4096 outputs of the tile.
 // The constants are a least-squares fit to timed launches.  On 2323 others
 // (MI355X, 120 random shapes of M 17..512, N 512..37888, K 1024..25600,
-// per-channel, gs 32 and 128, every tile and split; profiles/int4_plan_fit.md)
+// per-channel, gs 32 and 128, every tile and split)
 // the estimate is 0.5% high in the mean with an rms error of 10% (per-channel
 // 7% high, group-wise 4% low), and the tile and split it takes 2.5% off the
 // best at M <= 64, 1.4% up to M 128, 1.1% beyond, 13% at the worst.
